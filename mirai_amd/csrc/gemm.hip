@@ -129,7 +129,6 @@ struct Params {
   const int32_t *num_tiles;
   const int2 *tiles_r;       // dual launch: the 128-row remainder tiles
   const int32_t *num_tiles_r;
-  int slots_tall;            // dual launch: per-XCD slots of the 256-row tiles
   int stagger;               // dual launch: leading per-XCD slots given to remainder tiles
   const int64_t *seg_end;
   uint16_t *out;
@@ -1579,12 +1578,16 @@ void grouped_gemm_kernel(Params p) {
 }
 
 // 256-row tiles (p.tiles) and the 128-row remainder tiles (p.tiles_r) in one
-// launch. Each XCD runs its share of the tall tiles (slots p.stagger ..
-// p.stagger + p.slots_tall - 1, in the map above) and then the rest of its
-// share of the remainder tiles, which so fill the tail of the tall ones
-// instead of running as a launch of their own after it. The first p.stagger
-// slots of an XCD take remainder tiles: those CUs start their tall tiles half
-// a tile later, so the CUs' epilogues (the output stores) stop coinciding.
+// launch. Each XCD runs its share of the tall tiles (slots p.stagger onwards,
+// in the map above) and then the rest of its share of the remainder tiles,
+// which so fill the tail of the tall ones instead of running as a launch of
+// their own after it. The first p.stagger slots of an XCD take remainder
+// tiles: those CUs start their tall tiles half a tile later, so the CUs'
+// epilogues (the output stores) stop coinciding. The slots are cut by the
+// plan's counts, not by the launch's bounds, so the empty workgroups of a
+// launch all come last (with the tall slots cut by their bound, a launch of
+// few tall tiles first dispatched hundreds of empty workgroups: 2048 tokens,
+// top-8 of 128 experts, 397 against 382 us for the layer).
 template <int FMT, int EPI, bool LORA, class Tall, class Short>
 __global__ __launch_bounds__(Tall::NT) __attribute__((amdgpu_waves_per_eu(Tall::WAVES_PER_SIMD)))
 void grouped_gemm_dual_kernel(Params p) {
@@ -1598,25 +1601,20 @@ void grouped_gemm_dual_kernel(Params p) {
   __shared__ __attribute__((aligned(16))) uint8_t sLt[lora_tile_bytes<EPI, LORA, Tall>()];
   __shared__ float sCode[is_dq(FMT) ? 512 : 1];
   const int xcd = blockIdx.x & 7, slot = blockIdx.x >> 3;
-  const bool tall = slot >= p.stagger && slot < p.stagger + p.slots_tall;
-  if (tall) {
-    const int total = *p.num_tiles * p.n_tiles_n;
-    const int per_xcd = (total + 7) >> 3;
-    const int st = slot - p.stagger;
-    if (st >= per_xcd) return;
-    const int logical = xcd * per_xcd + st;
-    if (logical >= total) return;
+  const int total_t = *p.num_tiles * p.n_tiles_n, total_r = *p.num_tiles_r * p.n_tiles_n;
+  const int per_t = (total_t + 7) >> 3, per_r = (total_r + 7) >> 3;
+  const int stagger = min(p.stagger, per_r);
+  if (slot >= per_t + per_r) return;
+  if (slot >= stagger && slot < stagger + per_t) {
+    const int logical = xcd * per_t + slot - stagger;
+    if (logical >= total_t) return;
     const int mt = logical / p.n_tiles_n;
     load_code_tables<FMT>(p, sCode);
     gemm_tile<FMT, EPI, LORA, Tall>(p, p.tiles[mt], logical - mt * p.n_tiles_n, sA0, sA1, sB0,
                                     sB1, sLt, sCode);
   } else {
-    const int total = *p.num_tiles_r * p.n_tiles_n;
-    const int per_xcd = (total + 7) >> 3;
-    const int s2 = slot < p.stagger ? slot : slot - p.slots_tall;
-    if (s2 >= per_xcd) return;
-    const int logical = xcd * per_xcd + s2;
-    if (logical >= total) return;
+    const int logical = xcd * per_r + (slot < stagger ? slot : slot - per_t);
+    if (logical >= total_r) return;
     const int mt = logical / p.n_tiles_n;
     const int2 tile = p.tiles_r[mt];
     load_code_tables<FMT>(p, sCode);
@@ -1651,7 +1649,7 @@ int launch(const Params &p, int64_t max_row_tiles, hipStream_t s) {
 // The dual launch: room for max_tall 256-row tiles and max_short remainder
 // tiles (upper bounds; the kernel reads the plan's counts).
 template <int FMT, int EPI, bool LORA, class Tall, class Short>
-int launch_dual(Params p, int64_t max_tall, int64_t max_short, hipStream_t s) {
+int launch_dual(const Params &p, int64_t max_tall, int64_t max_short, hipStream_t s) {
   const int64_t slots_tall = ceil_div(max_tall * p.n_tiles_n, 8);
   const int64_t slots_short = ceil_div(max_short * p.n_tiles_n, 8);
   const int64_t grid = 8 * (slots_tall + slots_short);
@@ -1660,17 +1658,24 @@ int launch_dual(Params p, int64_t max_tall, int64_t max_short, hipStream_t s) {
     set_error("grouped GEMM grid too large");
     return MX_ERR_INVALID;
   }
-  p.slots_tall = static_cast<int>(slots_tall);
-  p.stagger = static_cast<int>(std::min<int64_t>(p.stagger, slots_short));
   hipLaunchKernelGGL((grouped_gemm_dual_kernel<FMT, EPI, LORA, Tall, Short>),
                      dim3(static_cast<unsigned>(grid)), dim3(Tall::NT), 0, s, p);
   return check_launch("grouped GEMM launch");
 }
 
-// Row-tile height: 256-row tiles when experts average at least 256 rows (the
-// taller tile's better MFMA / LDS ratio outweighs its tail waste from there
-// on, measured at C2, C3 and C5), else 128-row tiles.
-inline bool use_tall_tiles(int64_t rows, int experts) { return rows >= 256 * static_cast<int64_t>(experts); }
+// Row-tile height: the dual launch (256-row tiles, 128-row remainders) when
+// experts average at least 32 rows. An expert of up to 128 rows takes the same
+// 128-row tile in either launch, and one of 129 or more a tall tile, which
+// decodes its weights once where two 128-row tiles decode them twice: from 256
+// rows per expert down to 32 the dual launch was never slower (NF4 layer of 64
+// experts, 4095 tokens: 437 against 537 us; 2048: 328 against 351; 1024: even;
+// skewed top-8 of 128 experts, 512 tokens: 171 against 186). Below 32 few
+// experts exceed a 128-row tile, and the dual launch's empty workgroups cost
+// more (INT8, 300 tokens, 19 rows per expert: 463 against 484 us). The fp32
+// layer keeps 256: its down projection's K parts belong to the 128-row launch.
+inline bool use_tall_tiles(int fmt, int64_t rows, int experts) {
+  return rows >= (fmt == MX_FMT_F32X3 ? 256 : 32) * static_cast<int64_t>(experts);
+}
 
 // fp32 layer, down projection on 128-row tiles: K parts per tile, so that a
 // launch with few tiles (C1: at most 32 tiles of 48 K steps for 256 CUs)
@@ -1678,7 +1683,7 @@ inline bool use_tall_tiles(int64_t rows, int experts) { return rows >= 256 * sta
 // while the launch stays within one workgroup per CU.
 constexpr int kChipCUs = 256;
 inline int f32x3_down_parts(int64_t rows, int experts, int64_t hidden, int64_t ffn) {
-  if (use_tall_tiles(rows, experts)) return 1;
+  if (use_tall_tiles(MX_FMT_F32X3, rows, experts)) return 1;
   const int64_t slots = (ceil_div(rows, kPlanTileM) + experts) * ceil_div(hidden, 256);
   const int64_t steps = 3 * ffn / 64;
   int best = 1;
@@ -1687,7 +1692,7 @@ inline int f32x3_down_parts(int64_t rows, int experts, int64_t hidden, int64_t f
   return best;
 }
 
-// 128-row tiles only (experts averaging under 256 rows).
+// 128-row tiles only (use_tall_tiles).
 template <int EPI, bool LORA, class Short>
 int launch_tile(int fmt, const Params &p, int64_t max_tiles, hipStream_t s) {
   switch (fmt) {
@@ -1760,7 +1765,7 @@ int launch_fmt(int fmt, Params p, const PlanLayout &PL, const PlanView &v, bool 
   if (!tall) {
     p.tiles = v.tiles;
     p.num_tiles = v.num_tiles;
-    return launch_tile<EPI, LORA, Short>(fmt, p, PL.max_tiles, s);
+    return launch_tile<EPI, LORA, Short>(fmt, p, std::min(PL.max_tiles, PL.rows), s);
   }
   // 256-row tiles over each expert's rows except a final remainder of at most
   // 128 rows, which gets a 128-row tile (a short remainder costs about half a
@@ -1776,13 +1781,16 @@ int launch_fmt(int fmt, Params p, const PlanLayout &PL, const PlanView &v, bool 
   // then stop coinciding across the chip (C4 down -1.8 %). At about 2048 rows
   // per expert the gate/up GEMM gained nothing from it and lost 1.2 % at C4.
   p.stagger = (EPI == EPI_STORE || PL.rows < 1024 * static_cast<int64_t>(PL.experts)) ? 16 : 0;
-  return launch_tile_dual<EPI, LORA, Tall, Short>(fmt, p, PL.max_tiles2, PL.experts, s);
+  // A tall tile covers at least 129 rows of its expert, a remainder tile one.
+  const int64_t max_tall = std::min<int64_t>(PL.max_tiles2, PL.rows / (kPlanTileM + 1));
+  const int64_t max_short = std::min<int64_t>(PL.experts, PL.rows);
+  return launch_tile_dual<EPI, LORA, Tall, Short>(fmt, p, max_tall, max_short, s);
 }
 
 template <int EPI>
 int launch_any(int fmt, bool lora, const Params &p, const PlanLayout &PL, const PlanView &v,
                hipStream_t s) {
-  const bool tall = use_tall_tiles(PL.rows, PL.experts);
+  const bool tall = use_tall_tiles(fmt, PL.rows, PL.experts);
   return lora ? launch_fmt<EPI, true>(fmt, p, PL, v, tall, s)
               : launch_fmt<EPI, false>(fmt, p, PL, v, tall, s);
 }
