@@ -237,6 +237,18 @@ __device__ __forceinline__ int uniform_wave_index() {
   return __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
 }
 
+// Waits for the wave's outstanding LDS DMA (and vector loads). A barrier alone
+// publishes them to the other waves only where the compiler happens to wait
+// before it.
+__device__ __forceinline__ void wait_lds_dma() { __builtin_amdgcn_s_waitcnt(0x0f70); }  // vmcnt(0)
+
+// Swaps the upper 32 lanes of a with the lower 32 lanes of b (one instruction).
+__device__ __forceinline__ void swap_halves(uint32_t &a, uint32_t &b) {
+  const auto r = __builtin_amdgcn_permlane32_swap(a, b, false, false);
+  a = r[0];
+  b = r[1];
+}
+
 // Raw buffer over [base, base + bytes): accesses at offsets >= bytes are
 // dropped (stores) or read zero (loads) by the hardware range check. Tile
 // buffers stay far below 2 GiB.
@@ -1273,94 +1285,80 @@ __device__ __forceinline__ void gemm_tile(Params p, int2 tile, int nt, uint8_t *
   }
 }
 
-// ------------------------------------------------------------ light tiles
-// An expert with at most kLightRows rows in a launch (skewed routing leaves
-// many such) would pay a whole 128-row tile: the decode of its 256 x K weight
-// tile into LDS plus 128-row MFMA work, for a few rows. Its light tile keeps
-// the work per weight at one decode: all of the expert's token rows are staged
-// in LDS once (the four stage buffers, one barrier), and each wave decodes its
-// 32 weight rows straight into MFMA operands, each lane one whole 64-element
-// NF4 block per 128-wide K step, with no B stage and no per-step barrier.
-//
-// K permutation: in K step b a lane of half h (lane / 32) supplies, for MFMA
-// sub-step s, the 8 elements 128 b + 64 h + 8 s .. + 7 of its row, for the
-// weight operand and the token operand alike; the sum over K is the same sum.
-constexpr int kLightRows = 32;
+// ------------------------------------------------- weight-streaming tiles
+// Forward tiles of at most 128 rows (few rows per expert, remainders): the
+// weights are the work there, each is decoded once, and what bounds the tile
+// is the decode's VALU and the wait for the next weights, not MFMA. So each
+// wave decodes its own 32 weight rows straight into MFMA operands and holds
+// every row block's accumulators (MB = 1, 2 or 4 blocks of 32 rows): no B
+// stage, and one barrier per 128 columns of K, for the token rows that all
+// waves share through LDS. With 64 KB of LDS and 128 registers two workgroups
+// run on a CU, four waves per SIMD, and cover each other's waits; the tile that
+// stages decoded weights in LDS runs one, and a barrier per 64 columns.
+// Measured (kernel trace, hidden 2048, ffn 1408, 64 NF4 experts): gate/up at 256
+// tokens 82 -> 69 us (2.8 TB/s of packed weights), at 512 tokens 130 -> 80; INT8,
+// hidden 3072, ffn 2048, 300 tokens: the layer 474 -> 324 us (4.5 TB/s). Weights
+// loaded two or three steps ahead instead of one: slower (300 tokens INT8 324 ->
+// 348 us, 256 tokens NF4 163 -> 171).
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
+constexpr bool stream_format(int fmt) {
+  return fmt == MX_FMT_NF4 || fmt == MX_FMT_NF4_F32 || fmt == MX_FMT_NF4_DQ ||
+         fmt == MX_FMT_INT8 || fmt == MX_FMT_BF16;
+}
 template <int FMT, int EPI>
-constexpr bool light_capable() {
-  return (FMT == MX_FMT_NF4 || FMT == MX_FMT_NF4_F32 || FMT == MX_FMT_NF4_DQ) &&
-         (EPI == EPI_SWIGLU || EPI == EPI_STORE);
+constexpr bool stream_capable() {
+  return stream_format(FMT) && (EPI == EPI_SWIGLU || EPI == EPI_STORE);
+}
+// K columns per step: 128 (two NF4 blocks of a row, one per half-wave); bf16
+// weights take 64, so a lane's share of a step is 64 bytes.
+template <int FMT>
+constexpr int stream_kstep() {
+  return FMT == MX_FMT_BF16 ? 64 : 128;
 }
 
-// Columns of K the four stage buffers hold for 32 rows (two of SA bytes, two of SB).
-template <int SA, int SB>
-constexpr int light_max_k() {
-  return (2 * SA + 2 * SB) / (32 * 2);
-}
-
-// K in whole 128-wide steps (a lane takes one 64-block per step) that the
-// stage buffers hold.
-template <int SA, int SB>
-__device__ __forceinline__ bool light_tile_fits(const Params &p, int2 tile) {
-  return p.seg_end[tile.x] - tile.y <= kLightRows && p.K % 128 == 0 &&
-         p.K <= light_max_k<SA, SB>();
-}
-
-template <int FMT, int EPI, bool LORA, int SA, int SB>
-__device__ __forceinline__ void light_tile(const Params &p, int2 tile, int nt, uint8_t *sA0,
-                                           uint8_t *sA1, uint8_t *sB0, uint8_t *sB1,
-                                           const float *sCode) {
-  static_assert(SA % 8192 == 0 && SB % 8192 == 0, "stage rows must be whole 256-byte groups");
+template <int FMT, int EPI, bool LORA, int MB>
+__device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, uint8_t *sA0,
+                                            uint8_t *sA1, const float *sCode) {
+  constexpr int KS = stream_kstep<FMT>();
+  constexpr int SUB = KS / 16;          // MFMA steps per K step
+  constexpr int kRowsPerDma = 512 / KS; // token rows one DMA instruction fills
+  constexpr int kDmas = MB * 32 / kRowsPerDma;
+  constexpr int kMyDmas = (kDmas + 7) / 8;
   const int e = tile.x;
   const int64_t row0 = tile.y;
   const int64_t row_end = p.seg_end[e];
-  const int m = static_cast<int>(row_end - row0);  // 1 .. kLightRows
+  const int m = static_cast<int>(min(row_end - row0, static_cast<int64_t>(MB * 32)));
   const int wave = uniform_wave_index(), lane = threadIdx.x & 63;
-  const int K = static_cast<int>(p.K);
-  // Stage region q holds K columns [kq0, kq0 + kq) of the 32 rows, row stride
-  // 2 kq bytes, 16-byte chunks XOR-swizzled by (row & 15) inside each 256-byte
-  // group so the 32 rows a fragment read touches spread over the banks.
-  constexpr int kA = SA / 64, kB = SB / 64;  // K columns per region
-  auto region = [&](int q) __attribute__((always_inline)) -> uint8_t * {
-    return q == 0 ? sA0 : q == 1 ? sA1 : q == 2 ? sB0 : sB1;
-  };
-  auto region_k0 = [](int q) { return q < 2 ? q * kA : 2 * kA + (q - 2) * kB; };
-  auto region_k = [](int q) { return q < 2 ? kA : kB; };
+  const int li = lane & 31, h = lane >> 5;
 
   // ------------------------------------------- token rows -> LDS (by DMA)
-  // One DMA instruction fills 1 KB of a region (lane l at byte 16 l): rows of
-  // that region whose K range starts inside the layer's K. Rows past the
-  // segment are not loaded: they only feed output rows that are dropped.
-  {
+  // 16-byte chunks of a staged row XOR-ed with a row key, so the 32 rows of a
+  // fragment read spread over the banks. Rows past the segment re-read its
+  // last row: they only feed output rows that are dropped.
+  int a_row[kMyDmas], a_col[kMyDmas];
 #pragma unroll
-    for (int q = 0; q < 4; ++q) {
-      const int kq = region_k(q), kq0 = region_k0(q);
-      if (kq0 >= K) break;
-      const int rows_per_dma = 1024 / (2 * kq);  // 1 (kq = 512) or 2 (kq = 256)
-      const int n_dma = 32 / rows_per_dma;
-      for (int d = wave; d < n_dma; d += 8) {
-        if (d * rows_per_dma >= m) break;  // wave-uniform: the DMA's rows are past the segment
-        const int row = d * rows_per_dma + (lane * 16) / (2 * kq);
-        const int phys = ((lane * 16) % (2 * kq)) >> 4;
-        const int chunk = phys ^ (row & 15);
-        const int k = kq0 + 8 * chunk;
-        if (row < m && k < K) {
-          const int64_t sr = row0 + row;
-          const int64_t src = p.row_token ? static_cast<int64_t>(p.row_token[sr]) : sr;
-          __builtin_amdgcn_global_load_lds(
-              reinterpret_cast<const void *>(p.x + src * p.ldx + k),
-              reinterpret_cast<__attribute__((address_space(3))) void *>(
-                  reinterpret_cast<uintptr_t>(region(q) + d * 1024)),
-              16, 0, 0);
-        }
-      }
-    }
+  for (int i = 0; i < kMyDmas; ++i) {
+    const int row = (wave * kMyDmas + i) * kRowsPerDma + lane / (KS / 8);
+    const int phys = lane & (KS / 8 - 1);
+    a_col[i] = 8 * (phys ^ (KS == 64 ? swz_key64(row) : (row & 15)));
+    const int64_t sr = min(row0 + row, row_end - 1);
+    a_row[i] = p.row_token ? p.row_token[sr] : static_cast<int>(sr);
   }
+  auto load_a = [&](int b, uint8_t *sA) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < kMyDmas; ++i) {
+      const int d = wave * kMyDmas + i;
+      if (kDmas % 8 != 0 && d >= kDmas) break;  // wave-uniform
+      __builtin_amdgcn_global_load_lds(
+          reinterpret_cast<const void *>(p.x + a_row[i] * p.ldx + (b * KS + a_col[i])),
+          reinterpret_cast<__attribute__((address_space(3))) void *>(
+              reinterpret_cast<uintptr_t>(sA + d * 1024)),
+          16, 0, 0);
+    }
+  };
 
   // ----------------------------------------------------- the wave's weights
-  const int li = lane & 31, h = lane >> 5;
   int which = 0;
   int64_t n;
   if (EPI == EPI_SWIGLU) {
@@ -1374,10 +1372,24 @@ __device__ __forceinline__ void light_tile(const Params &p, int2 tile, int nt, u
   }
   const int64_t n_row = min(n, p.N - 1);  // rows past N feed dropped columns
   const int64_t wrow = static_cast<int64_t>(e) * pick(p.wn, which) + n_row;
-  const uint8_t *codes = static_cast<const uint8_t *>(pick(p.w, which)) + wrow * (p.K / 2);
-  const uint8_t *absrow = static_cast<const uint8_t *>(pick(p.wscale, which)) +
-                          wrow * (p.K / kNf4Block) * absmax_bytes(FMT);
-  // NF4_DQ: the row's nested scales (K <= 2048 here: at most two groups).
+  // Bytes of one lane's share of a step, its 16-byte registers and the row's
+  // bytes per step.
+  constexpr int kLaneBytes = is_nf4(FMT) ? KS / 4 : FMT == MX_FMT_INT8 ? KS / 2 : KS;
+  constexpr int kQ = kLaneBytes / 16;
+  // bf16: a lane's 16-byte pieces lie 32 bytes apart (MFMA step s, half h at
+  // 32 s + 16 h); the others take kLaneBytes in a row and exchange halves.
+  constexpr int kPiece = FMT == MX_FMT_BF16 ? 32 : 16;
+  const uint8_t *codes = static_cast<const uint8_t *>(pick(p.w, which)) +
+                         wrow * (p.K * (2 * kLaneBytes) / KS) +
+                         h * (FMT == MX_FMT_BF16 ? 16 : kLaneBytes);
+  const uint8_t *absrow = nullptr;
+  float i8_scale = 0.0f;
+  if constexpr (is_nf4(FMT))
+    absrow = static_cast<const uint8_t *>(pick(p.wscale, which)) +
+             wrow * (p.K / kNf4Block) * absmax_bytes(FMT);
+  if constexpr (FMT == MX_FMT_INT8)
+    i8_scale = bf16_bits_to_f32(static_cast<const uint16_t *>(pick(p.wscale, which))[wrow]);
+  // NF4_DQ: the row's nested scales (K <= 16384: at most two groups).
   float dq_lo = 0.0f, dq_hi = 0.0f, dq_off = 0.0f;
   int dq_sw = 0;
   if constexpr (is_dq(FMT)) {
@@ -1388,79 +1400,147 @@ __device__ __forceinline__ void light_tile(const Params &p, int2 tile, int nt, u
     dq_sw = static_cast<int>((((b0 >> 8) + 1) << 8) - b0);
     dq_off = pick2(p.dq_offset, which)[e];
   }
-  const int KS = K / 128;  // K steps
   struct Codes {
-    u32x4 q[2];
+    u32x4 q[kQ];
     uint32_t abs;
   };
   auto load_codes = [&](int b, Codes &c) __attribute__((always_inline)) {
-    const int blk = 2 * b + h;
-    c.q[0] = *reinterpret_cast<const u32x4 *>(codes + blk * 32);
-    c.q[1] = *reinterpret_cast<const u32x4 *>(codes + blk * 32 + 16);
-    c.abs = load_absmax<FMT>(absrow, blk);
+#pragma unroll
+    for (int q = 0; q < kQ; ++q)
+      c.q[q] = *reinterpret_cast<const u32x4 *>(codes + static_cast<int64_t>(b) * (2 * kLaneBytes) + kPiece * q);
+    c.abs = is_nf4(FMT) ? load_absmax<FMT>(absrow, 2 * b + h) : 0u;
   };
 
-  f32x16 acc;
+  f32x16 acc[MB];
 #pragma unroll
-  for (int j = 0; j < 16; ++j) acc[j] = 0.0f;
-  Codes c0, c1;
-  load_codes(0, c0);
-  __syncthreads();  // the staged token rows of every wave
+  for (int mb = 0; mb < MB; ++mb)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) acc[mb][j] = 0.0f;
 
-  auto kstep = [&](int b, const Codes &c) __attribute__((always_inline)) {
-    const int k = 128 * b + 64 * h;
-    int q = 0;
-#pragma unroll
-    for (int r = 1; r < 4; ++r) q += k >= region_k0(r) ? 1 : 0;
-    const int kq = region_k(q);
-    const uint8_t *arow = region(q) + li * (2 * kq);
-    const int c0k = (k - region_k0(q)) >> 3;  // first 16-byte chunk of the lane's 64 elements
-    Nf4Table t;
-    if constexpr (is_dq(FMT)) {
-      const int blk = 2 * b + h;
-      t = nf4_table(dq_absmax(sCode[which * 256 + c.abs], blk < dq_sw ? dq_lo : dq_hi, dq_off));
-    } else {
-      t = nf4_table(absmax_value<FMT>(c.abs));
+  // The lane's fragment of MFMA step s in row block 0: chunk 2 s + h of row
+  // li, at frag0 ^ (s << 5) (h has no bit of 2 s; blocks of 32 rows repeat the
+  // row key).
+  int frag0 = li * (2 * KS) + ((h ^ (KS == 64 ? swz_key64(li) : (li & 15))) << 4);
+  // One K step on stage `cur`: the barrier publishes its rows (loaded during
+  // the step before) and frees the other stage, whose next rows and the next
+  // codes then load while this step multiplies.
+  const int nb = static_cast<int>(p.K) / KS;
+  auto step = [&](int b, const uint8_t *cur, uint8_t *nxt, const Codes &cc, Codes &cn)
+      __attribute__((always_inline)) {
+    wait_lds_dma();
+    __syncthreads();
+    if (b + 1 < nb) {
+      load_a(b + 1, nxt);
+      load_codes(b + 1, cn);
     }
+    // Opaque, so that the fragment addresses are formed where they are used
+    // (one XOR each) instead of held in registers over the loop.
+    asm volatile("" : "+v"(frag0));
+    // The step's 128 K columns are two 64-blocks of the row, block h loaded by
+    // half h. The MFMA takes K in natural order (half h: columns 16 s + 8 h ..
+    // + 7, as every other tile, so a row's sum has the same bits whichever
+    // tile runs it): the halves swap every second group of 8, after which both
+    // hold their columns of block 0 in the even groups and of block 1 in the
+    // odd ones. Of the NF4 blocks either the decode tables are swapped likewise
+    // (t0, t1), or, where the accumulators leave no registers for two tables,
+    // the absmax values (abs0, abs1), and each table is built when its block
+    // begins.
+    constexpr bool kSwapTables = MB <= 2;
+    constexpr int kGroup = is_nf4(FMT) ? 1 : 2;  // dwords per group of 8 weights
+    uint32_t w[4 * kQ];
 #pragma unroll
-    for (int s = 0; s < 8; ++s) {
-      const int chunk = c0k + s;
-      const int phys = (chunk & ~15) | ((chunk & 15) ^ (li & 15));
-      const bf16x8 a = *reinterpret_cast<const bf16x8 *>(arow + phys * 16);
+    for (int q = 0; q < 4 * kQ; ++q) w[q] = cc.q[q >> 2][q & 3];
+    float abs0 = 0.0f, abs1 = 0.0f;
+    if constexpr (KS == 128) {
+#pragma unroll
+      for (int g = 0; g < 8; g += 2)
+#pragma unroll
+        for (int q = 0; q < kGroup; ++q) swap_halves(w[kGroup * g + q], w[kGroup * (g + 1) + q]);
+    }
+    Nf4Table t0 = {}, t1 = {};
+    if constexpr (is_nf4(FMT)) {
+      float av;
+      if constexpr (is_dq(FMT))
+        av = dq_absmax(sCode[which * 256 + cc.abs], 2 * b + h < dq_sw ? dq_lo : dq_hi, dq_off);
+      else
+        av = absmax_value<FMT>(cc.abs);
+      if constexpr (kSwapTables) {
+        t0 = t1 = nf4_table(av);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          swap_halves(t0.lo[j], t1.lo[j]);
+          swap_halves(t0.hi[j], t1.hi[j]);
+        }
+      } else {
+        uint32_t a0 = __float_as_uint(av), a1 = a0;
+        swap_halves(a0, a1);
+        abs0 = __uint_as_float(a0);
+        abs1 = __uint_as_float(a1);
+      }
+    }
+    Nf4Table t = {};
+#pragma unroll
+    for (int s = 0; s < SUB; ++s) {
+      if constexpr (is_nf4(FMT)) {
+        if (kSwapTables)
+          t = s < SUB / 2 ? t0 : t1;
+        else if (s % (SUB / 2) == 0)
+          t = nf4_table(s == 0 ? abs0 : abs1);
+      }
+      bf16x8 a[MB];
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+        a[mb] = *reinterpret_cast<const bf16x8 *>(cur + (frag0 ^ (s << 5)) + 32 * mb * (2 * KS));
+      // Group of MFMA step s: the even ones of block 0, then the odd ones.
+      const int g = 2 * (s & 3) + (s >> 2);
       uint32_t d[4];
-      const u32x4 v = c.q[s >> 2];
-      const uint32_t word = (s & 3) == 0 ? v[0] : (s & 3) == 1 ? v[1] : (s & 3) == 2 ? v[2] : v[3];
-      nf4_decode8(t, word, d);
-      const bf16x8 w = __builtin_bit_cast(bf16x8, u32x4{d[0], d[1], d[2], d[3]});
-      acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(w, a, acc, 0, 0, 0);
+      if constexpr (is_nf4(FMT)) {
+        nf4_decode8(t, w[g], d);
+      } else if constexpr (FMT == MX_FMT_INT8) {
+#pragma unroll
+        for (int u = 0; u < 2; ++u) {
+          const uint32_t v = w[2 * g + u];
+          d[2 * u] = pack_bf16x2(sbyte_to_f32<0>(v) * i8_scale, sbyte_to_f32<1>(v) * i8_scale);
+          d[2 * u + 1] = pack_bf16x2(sbyte_to_f32<2>(v) * i8_scale, sbyte_to_f32<3>(v) * i8_scale);
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < 4; ++u) d[u] = w[4 * s + u];
+      }
+      const bf16x8 wf = __builtin_bit_cast(bf16x8, u32x4{d[0], d[1], d[2], d[3]});
+#pragma unroll
+      for (int mb = 0; mb < MB; ++mb)
+        acc[mb] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(wf, a[mb], acc[mb], 0, 0, 0);
     }
   };
-  // The codes of step b + 1 load while step b decodes.
+  Codes c0, c1;
+  load_a(0, sA0);
+  load_codes(0, c0);
   int b = 0;
-  for (; b + 1 < KS; b += 2) {
-    load_codes(b + 1, c1);
-    kstep(b, c0);
-    load_codes(min(b + 2, KS - 1), c0);
-    kstep(b + 1, c1);
+  for (; b + 1 < nb; b += 2) {
+    step(b, sA0, sA1, c0, c1);
+    step(b + 1, sA1, sA0, c1, c0);
   }
-  if (b < KS) kstep(b, c0);
+  if (b < nb) step(b, sA0, sA1, c0, c1);
 
-  // --------------------------------------------------- LoRA up-projection
-  // The low-rank row holds [gate rc | up rc] (SwiGLU) or the down adapter's
-  // rc columns; one MFMA chain over them with each lane's factor row zero
-  // outside its own adapter gives the gate and up deltas of the block apart.
-  const int lrow = li;
-  const int64_t prow_i = min(row0 + lrow, row_end - 1);
-  f32x16 lacc;
+  // Per row block: the LoRA up-projection, one MFMA chain per adapter. For
+  // SwiGLU both chains run over all 32 weight rows of the wave, each lane with
+  // its own column's factor row of the chain's adapter; the gate chain's up
+  // rows (and the reverse) are not read. Then the epilogue: value v of a lane
+  // is output row lane % 32 of the block and weight row 8 (v / 4) + 4 h + v % 4.
+  constexpr int n_ad = EPI == EPI_SWIGLU ? 2 : 1;
 #pragma unroll
-  for (int j = 0; j < 16; ++j) lacc[j] = 0.0f;
-  if (LORA) {
-    constexpr int n_ad = EPI == EPI_SWIGLU ? 2 : 1;
+  for (int mb = 0; mb < MB; ++mb) {
+    const int lrow = 32 * mb + li;
+    f32x16 lacc[n_ad];
 #pragma unroll
     for (int ad = 0; ad < n_ad; ++ad) {
+#pragma unroll
+      for (int j = 0; j < 16; ++j) lacc[ad][j] = 0.0f;
+      if (!LORA) continue;
       const int r = pick2(p.lora_r, ad);
       if (r == 0) continue;
-      const bool own = EPI == EPI_SWIGLU ? (which == ad) : true;
+      const int64_t prow_i = min(row0 + lrow, row_end - 1);
       const uint16_t *frow = pick2(p.lora_b, ad) + (static_cast<int64_t>(e) * p.N + n_row) * r;
       const uint16_t *arow = p.lora_p + prow_i * p.ldp + ad * p.lora_rc;
       for (int c = 0; c < r; c += 16) {
@@ -1468,59 +1548,67 @@ __device__ __forceinline__ void light_tile(const Params &p, int2 tile, int nt, u
         // Columns past the rank hold zero activations; their factor read
         // stays inside the row.
         const bf16x8 a = *reinterpret_cast<const bf16x8 *>(arow + col);
-        bf16x8 f = *reinterpret_cast<const bf16x8 *>(frow + (col < r ? col : 0));
-        if (!own) f = __builtin_bit_cast(bf16x8, u32x4{0u, 0u, 0u, 0u});
-        lacc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, a, lacc, 0, 0, 0);
+        const bf16x8 f = *reinterpret_cast<const bf16x8 *>(frow + (col < r ? col : 0));
+        lacc[ad] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, a, lacc[ad], 0, 0, 0);
       }
     }
-  }
-
-  // ------------------------------------------------------------ epilogue
-  // Value v of a lane is output row lane % 32 of the block and block row
-  // 8 (v / 4) + 4 h + v % 4: runs of 4 consecutive columns.
-  if (lrow >= m) return;
-  if (EPI == EPI_SWIGLU) {
-    const int64_t r = row0 + lrow;
+    if (lrow >= m) continue;
+    if (EPI == EPI_SWIGLU) {
+      const int64_t r = row0 + lrow;
 #pragma unroll
-    for (int g = 0; g < 2; ++g) {
-      const int64_t f0 = static_cast<int64_t>(nt) * 128 + 16 * wave + 8 * g + 4 * h;
-      float gv[4], uv[4], a[4], bb[4];
+      for (int g = 0; g < 2; ++g) {
+        const int64_t f0 = static_cast<int64_t>(nt) * 128 + 16 * wave + 8 * g + 4 * h;
+        float gv[4], uv[4], a[4], bb[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        gv[q] = acc[4 * g + q];
-        uv[q] = acc[8 + 4 * g + q];
-        a[q] = LORA ? lacc[4 * g + q] : 0.0f;
-        bb[q] = LORA ? lacc[8 + 4 * g + q] : 0.0f;
-      }
-      uint32_t h0, h1;
-      gated_run<LORA>(gv, uv, a, bb, p.act, h0, h1);
-      if (f0 < p.N) {
-        *reinterpret_cast<u32x2 *>(p.out + r * p.ldo + f0) = u32x2{h0, h1};
-        if (p.save_gate != nullptr) {
-          *reinterpret_cast<u32x2 *>(p.save_gate + r * p.N + f0) =
-              u32x2{pack_bf16x2(gv[0], gv[1]), pack_bf16x2(gv[2], gv[3])};
-          *reinterpret_cast<u32x2 *>(p.save_up + r * p.N + f0) =
-              u32x2{pack_bf16x2(uv[0], uv[1]), pack_bf16x2(uv[2], uv[3])};
+        for (int q = 0; q < 4; ++q) {
+          gv[q] = acc[mb][4 * g + q];
+          uv[q] = acc[mb][8 + 4 * g + q];
+          a[q] = LORA ? lacc[0][4 * g + q] : 0.0f;
+          bb[q] = LORA ? lacc[n_ad - 1][8 + 4 * g + q] : 0.0f;
+        }
+        uint32_t h0, h1;
+        gated_run<LORA>(gv, uv, a, bb, p.act, h0, h1);
+        if (f0 < p.N) {
+          *reinterpret_cast<u32x2 *>(p.out + r * p.ldo + f0) = u32x2{h0, h1};
+          if (p.save_gate != nullptr) {
+            *reinterpret_cast<u32x2 *>(p.save_gate + r * p.N + f0) =
+                u32x2{pack_bf16x2(gv[0], gv[1]), pack_bf16x2(gv[2], gv[3])};
+            *reinterpret_cast<u32x2 *>(p.save_up + r * p.N + f0) =
+                u32x2{pack_bf16x2(uv[0], uv[1]), pack_bf16x2(uv[2], uv[3])};
+          }
         }
       }
-    }
-  } else {
-    const int64_t sr = row0 + lrow;
-    const int64_t o = p.out_row ? static_cast<int64_t>(p.out_row[sr]) : sr;
+    } else {
+      const int64_t sr = row0 + lrow;
+      const int64_t o = p.out_row ? static_cast<int64_t>(p.out_row[sr]) : sr;
 #pragma unroll
-    for (int g = 0; g < 4; ++g) {
-      const int64_t n0 = static_cast<int64_t>(nt) * 256 + 32 * wave + 8 * g + 4 * h;
-      float v[4], a[4];
+      for (int g = 0; g < 4; ++g) {
+        const int64_t n0 = static_cast<int64_t>(nt) * 256 + 32 * wave + 8 * g + 4 * h;
+        float v[4], a[4];
 #pragma unroll
-      for (int q = 0; q < 4; ++q) {
-        v[q] = acc[4 * g + q];
-        a[q] = LORA ? lacc[4 * g + q] : 0.0f;
+        for (int q = 0; q < 4; ++q) {
+          v[q] = acc[mb][4 * g + q];
+          a[q] = LORA ? lacc[0][4 * g + q] : 0.0f;
+        }
+        uint32_t w0, w1;
+        projection_run<LORA>(v, a, w0, w1);
+        if (n0 < p.N) *reinterpret_cast<u32x2 *>(p.out + o * p.ldo + n0) = u32x2{w0, w1};
       }
-      uint32_t w0, w1;
-      projection_run<LORA>(v, a, w0, w1);
-      if (n0 < p.N) *reinterpret_cast<u32x2 *>(p.out + o * p.ldo + n0) = u32x2{w0, w1};
     }
   }
+}
+
+// The tile's rows in the fewest row blocks.
+template <int FMT, int EPI, bool LORA>
+__device__ __forceinline__ void stream_rows(const Params &p, int2 tile, int nt, uint8_t *sA0,
+                                            uint8_t *sA1, const float *sCode) {
+  const int64_t m = p.seg_end[tile.x] - tile.y;
+  if (m <= 32)
+    stream_tile<FMT, EPI, LORA, 1>(p, tile, nt, sA0, sA1, sCode);
+  else if (m <= 64)
+    stream_tile<FMT, EPI, LORA, 2>(p, tile, nt, sA0, sA1, sCode);
+  else
+    stream_tile<FMT, EPI, LORA, 4>(p, tile, nt, sA0, sA1, sCode);
 }
 
 // NF4_DQ: the code tables of the launch's weights (w[0], w[1]) into LDS,
@@ -1544,13 +1632,8 @@ __device__ __forceinline__ void load_code_tables(const Params &p, float *sCode) 
 template <int FMT, int EPI, bool LORA, class T>
 __global__ __launch_bounds__(T::NT) __attribute__((amdgpu_waves_per_eu(T::WAVES_PER_SIMD)))
 void grouped_gemm_kernel(Params p) {
-  // 128-row tiles of the layer GEMMs: A stages of 32 KB, so that the light
-  // tile stages up to 2048 K columns (the kernel runs one workgroup per CU
-  // by its registers, so the LDS costs no occupancy).
-  constexpr bool kLight = light_capable<FMT, EPI>() && T::BM == 128;
-  constexpr int kStageA = kLight && T::STAGE_A < 32768 ? 32768 : T::STAGE_A;
-  __shared__ __attribute__((aligned(16))) uint8_t sA0[kStageA];
-  __shared__ __attribute__((aligned(16))) uint8_t sA1[kStageA];
+  __shared__ __attribute__((aligned(16))) uint8_t sA0[T::STAGE_A];
+  __shared__ __attribute__((aligned(16))) uint8_t sA1[T::STAGE_A];
   __shared__ __attribute__((aligned(16))) uint8_t sB0[T::STAGE_B];
   __shared__ __attribute__((aligned(16))) uint8_t sB1[T::STAGE_B];
   __shared__ __attribute__((aligned(16))) uint8_t sLt[lora_tile_bytes<EPI, LORA, T>()];
@@ -1566,15 +1649,42 @@ void grouped_gemm_kernel(Params p) {
   const int mt = logical / p.n_tiles_n;
   const int2 tile = p.tiles[mt];
   load_code_tables<FMT>(p, sCode);
-  if constexpr (kLight) {
-    if (light_tile_fits<kStageA, T::STAGE_B>(p, tile)) {
-      light_tile<FMT, EPI, LORA, kStageA, T::STAGE_B>(p, tile, logical - mt * p.n_tiles_n, sA0,
-                                                      sA1, sB0, sB1, sCode);
-      return;
-    }
-  }
   gemm_tile<FMT, EPI, LORA, T>(p, tile, logical - mt * p.n_tiles_n, sA0, sA1, sB0, sB1, sLt, sCode,
                                part);
+}
+
+// Weight-streaming launch: 128-row tiles (p.tiles), 256 weight rows per
+// workgroup, the tile map of grouped_gemm_kernel.
+template <int FMT, int EPI, bool LORA>
+__global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
+void stream_gemm_kernel(Params p) {
+  constexpr int kStage = kPlanTileM * stream_kstep<FMT>() * 2;
+  __shared__ __attribute__((aligned(16))) uint8_t sA0[kStage];
+  __shared__ __attribute__((aligned(16))) uint8_t sA1[kStage];
+  __shared__ float sCode[is_dq(FMT) ? 512 : 1];
+  const int total = *p.num_tiles * p.n_tiles_n;
+  const int per_xcd = (total + 7) >> 3;
+  const int slot = blockIdx.x >> 3;
+  if (slot >= per_xcd) return;
+  const int job = (blockIdx.x & 7) * per_xcd + slot;
+  if (job >= total) return;
+  const int mt = job / p.n_tiles_n, nt = job - mt * p.n_tiles_n;
+  const int2 tile = p.tiles[mt];
+  load_code_tables<FMT>(p, sCode);
+  stream_rows<FMT, EPI, LORA>(p, tile, nt, sA0, sA1, sCode);
+}
+
+template <int FMT, int EPI, bool LORA>
+int launch_stream(const Params &p, int64_t max_tiles, hipStream_t s) {
+  const int64_t grid = 8 * ceil_div(max_tiles * p.n_tiles_n, 8);
+  if (grid <= 0) return MX_OK;
+  if (grid > 0x7fffffff) {
+    set_error("grouped GEMM grid too large");
+    return MX_ERR_INVALID;
+  }
+  hipLaunchKernelGGL((stream_gemm_kernel<FMT, EPI, LORA>), dim3(static_cast<unsigned>(grid)),
+                     dim3(512), 0, s, p);
+  return check_launch("grouped GEMM launch");
 }
 
 // 256-row tiles (p.tiles) and the 128-row remainder tiles (p.tiles_r) in one
@@ -1618,11 +1728,11 @@ void grouped_gemm_dual_kernel(Params p) {
     const int mt = logical / p.n_tiles_n;
     const int2 tile = p.tiles_r[mt];
     load_code_tables<FMT>(p, sCode);
-    // An expert's only tile, when it has at most kLightRows rows.
-    if constexpr (light_capable<FMT, EPI>()) {
-      if (light_tile_fits<Tall::STAGE_A, Tall::STAGE_B>(p, tile)) {
-        light_tile<FMT, EPI, LORA, Tall::STAGE_A, Tall::STAGE_B>(p, tile, logical - mt * p.n_tiles_n,
-                                                               sA0, sA1, sB0, sB1, sCode);
+    // The forward's remainder tiles stream their weights too (top-8 of 128
+    // experts, skewed: 8192 tokens 896 -> 878 us, INT8 3000 tokens 730 -> 682).
+    if constexpr (stream_capable<FMT, EPI>()) {
+      if (p.K % 128 == 0) {
+        stream_rows<FMT, EPI, LORA>(p, tile, logical - mt * p.n_tiles_n, sA0, sA1, sCode);
         return;
       }
     }
@@ -1663,18 +1773,30 @@ int launch_dual(const Params &p, int64_t max_tall, int64_t max_short, hipStream_
   return check_launch("grouped GEMM launch");
 }
 
-// Row-tile height: the dual launch (256-row tiles, 128-row remainders) when
-// experts average at least 32 rows. An expert of up to 128 rows takes the same
-// 128-row tile in either launch, and one of 129 or more a tall tile, which
-// decodes its weights once where two 128-row tiles decode them twice: from 256
-// rows per expert down to 32 the dual launch was never slower (NF4 layer of 64
-// experts, 4095 tokens: 437 against 537 us; 2048: 328 against 351; 1024: even;
-// skewed top-8 of 128 experts, 512 tokens: 171 against 186). Below 32 few
-// experts exceed a 128-row tile, and the dual launch's empty workgroups cost
-// more (INT8, 300 tokens, 19 rows per expert: 463 against 484 us). The fp32
-// layer keeps 256: its down projection's K parts belong to the 128-row launch.
-inline bool use_tall_tiles(int fmt, int64_t rows, int experts) {
-  return rows >= (fmt == MX_FMT_F32X3 ? 256 : 32) * static_cast<int64_t>(experts);
+// Whether a launch takes the dual kernel (256-row tiles, remainders of at most
+// 128 rows) or 128-row tiles alone: by the rows per expert on average.
+// * The forward over NF4, INT8 and bf16 weights (`stream`): the 128-row tiles
+//   are weight-streaming tiles at two workgroups per CU. Layers of 64 or 128
+//   experts, streaming against dual: INT8 at 24 rows per expert 328 / 369 us, 48
+//   382 / 412, 56 458 / 439; NF4 at 32 182 / 248, at 64 247 / 263 with even
+//   routes but 265 / 242 skewed (heavy experts want tall tiles): 48. bf16
+//   weights are four times the bytes to wait for, and the second workgroup
+//   pays longer: at 80 344 / 374, at 112 409 / 409. With few K steps a tile is
+//   mostly its start and end, which the second workgroup covers: K = 256 and
+//   512, 256 experts, at 150 142 / 161, 256 196 / 210, INT8 at 300 242 / 236.
+// * Otherwise both launches cover up to 128 rows with the same tile, and a
+//   tall tile decodes the weights of 129 or more rows once instead of twice:
+//   from 32 rows per expert on the dual launch was never slower, below that few
+//   experts exceed 128 rows and its empty workgroups cost more.
+// * The fp32 layer keeps 256: its down projection's K parts belong to the
+//   128-row launch.
+inline bool use_tall_tiles(int fmt, bool stream, int64_t K, int64_t rows, int experts) {
+  const int64_t least = fmt == MX_FMT_F32X3  ? 256
+                        : !stream            ? 32
+                        : K <= 512           ? 256
+                        : fmt == MX_FMT_BF16 ? 112
+                                             : 48;
+  return rows >= least * static_cast<int64_t>(experts);
 }
 
 // fp32 layer, down projection on 128-row tiles: K parts per tile, so that a
@@ -1683,7 +1805,7 @@ inline bool use_tall_tiles(int fmt, int64_t rows, int experts) {
 // while the launch stays within one workgroup per CU.
 constexpr int kChipCUs = 256;
 inline int f32x3_down_parts(int64_t rows, int experts, int64_t hidden, int64_t ffn) {
-  if (use_tall_tiles(MX_FMT_F32X3, rows, experts)) return 1;
+  if (use_tall_tiles(MX_FMT_F32X3, false, 3 * ffn, rows, experts)) return 1;
   const int64_t slots = (ceil_div(rows, kPlanTileM) + experts) * ceil_div(hidden, 256);
   const int64_t steps = 3 * ffn / 64;
   int best = 1;
@@ -1753,7 +1875,25 @@ int launch_tile_dual(int fmt, const Params &p, int64_t max_tall, int64_t max_sho
 }
 
 template <int EPI, bool LORA>
-int launch_fmt(int fmt, Params p, const PlanLayout &PL, const PlanView &v, bool tall, hipStream_t s) {
+int launch_stream_fmt(int fmt, const Params &p, int64_t max_tiles, hipStream_t s) {
+  switch (fmt) {
+    case MX_FMT_BF16:
+      return launch_stream<MX_FMT_BF16, EPI, LORA>(p, max_tiles, s);
+    case MX_FMT_NF4:
+      return launch_stream<MX_FMT_NF4, EPI, LORA>(p, max_tiles, s);
+    case MX_FMT_NF4_F32:
+      return launch_stream<MX_FMT_NF4_F32, EPI, LORA>(p, max_tiles, s);
+    case MX_FMT_NF4_DQ:
+      return launch_stream<MX_FMT_NF4_DQ, EPI, LORA>(p, max_tiles, s);
+    case MX_FMT_INT8:
+      return launch_stream<MX_FMT_INT8, EPI, LORA>(p, max_tiles, s);
+  }
+  set_error("unknown weight format %d", fmt);
+  return MX_ERR_INVALID;
+}
+
+template <int EPI, bool LORA>
+int launch_fmt(int fmt, Params p, const PlanLayout &PL, const PlanView &v, hipStream_t s) {
   // Column tiles are 256 wide (EPI_SWIGLU: 128 ffn columns of gate and of up).
   // The forward down projection (store epilogue) runs faster with its 8
   // waves as 4 x 2 (64 x 128 per wave); the others as 2 x 4 (measured).
@@ -1761,11 +1901,16 @@ int launch_fmt(int fmt, Params p, const PlanLayout &PL, const PlanView &v, bool 
                                          Tile<256, 256, 2, 4, 64>>::type;
   using Short = Tile<128, 256, 2, 4, 64>;
   p.n_tiles_n = static_cast<int>(EPI == EPI_SWIGLU ? ceil_div(p.N, 128) : ceil_div(p.N, 256));
+  const bool stream = EPI != EPI_STORE2 && stream_format(fmt) && p.K % 128 == 0;
+  bool tall = use_tall_tiles(fmt, stream, p.K, PL.rows, PL.experts);
   if (EPI == EPI_STORE2 && (fmt == MX_FMT_NF4_DQ || fmt == MX_FMT_NF4_DQ_KN)) tall = false;
   if (!tall) {
     p.tiles = v.tiles;
     p.num_tiles = v.num_tiles;
-    return launch_tile<EPI, LORA, Short>(fmt, p, std::min(PL.max_tiles, PL.rows), s);
+    const int64_t max_tiles = std::min(PL.max_tiles, PL.rows);
+    if constexpr (EPI == EPI_SWIGLU || EPI == EPI_STORE)
+      if (stream) return launch_stream_fmt<EPI, LORA>(fmt, p, max_tiles, s);
+    return launch_tile<EPI, LORA, Short>(fmt, p, max_tiles, s);
   }
   // 256-row tiles over each expert's rows except a final remainder of at most
   // 128 rows, which gets a 128-row tile (a short remainder costs about half a
@@ -1790,9 +1935,7 @@ int launch_fmt(int fmt, Params p, const PlanLayout &PL, const PlanView &v, bool 
 template <int EPI>
 int launch_any(int fmt, bool lora, const Params &p, const PlanLayout &PL, const PlanView &v,
                hipStream_t s) {
-  const bool tall = use_tall_tiles(fmt, PL.rows, PL.experts);
-  return lora ? launch_fmt<EPI, true>(fmt, p, PL, v, tall, s)
-              : launch_fmt<EPI, false>(fmt, p, PL, v, tall, s);
+  return lora ? launch_fmt<EPI, true>(fmt, p, PL, v, s) : launch_fmt<EPI, false>(fmt, p, PL, v, s);
 }
 
 // ------------------------------------------------------------ host helpers

@@ -69,3 +69,48 @@ def test_rows_around_the_tile_heights_backward(case):
     _, ref = _oracle_grads(w, dense, lora, x, scores, idx, dy, torch.arange(w.tokens))
     for name, e in ref.items():
         _close(name, g[name], e)
+
+
+# Streaming tiles: one, two and four row blocks of 32, each at its edges; 640
+# and 384 K columns take the rules of long and of short K, 192 is no multiple
+# of a streaming step (128) and keeps the tiles that stage decoded weights.
+STREAM_COUNTS = (1, 31, 32, 33, 0, 64, 65, 97, 128, 2, 0, 0)
+
+
+@pytest.mark.parametrize("rank", [0, 16, 40])
+@pytest.mark.parametrize("d,f", [(640, 384), (128, 320), (192, 256)])
+@pytest.mark.parametrize("fmt", ["nf4", "int8", "bf16"])
+def test_streaming_tiles(fmt, d, f, rank):
+    w = workload(fmt, STREAM_COUNTS, d=d, f=f, r=max(rank, 1))
+    idx, scores = exact_routes(STREAM_COUNTS, 7)
+    dense, x = wl.dense_weights(w), wl.tokens(w)
+    lora = wl.lora_factors(w) if rank else None
+    m = build_module(w, dense, lora)
+    with torch.no_grad():
+        out = m.run_direct_routed(x.cuda(), scores.cuda(), idx.cuda())
+    ref = olayer.layer_forward(x, scores, idx, oracle_weights(w, dense), oracle_loras(w, lora),
+                               w.experts)
+    assert_layer_close(out.cpu(), ref)
+
+
+@pytest.mark.parametrize("fmt", ["nf4", "int8", "bf16"])
+def test_a_rows_bits_do_not_depend_on_the_launch(fmt):
+    # The same rows of experts 0 .. 10 alone (streaming launch) and beside a
+    # heavy expert 11 (the launch with 256-row tiles), and the heavy expert's
+    # rows in 300s (256 + 44) and in 100s: every tile sums K in one order.
+    w = workload(fmt, STREAM_COUNTS, d=640, f=384)
+    m = build_module(w, wl.dense_weights(w), wl.lora_factors(w))
+    x = wl.tokens(w.with_tokens(w.tokens + 900)).cuda()
+    idx = torch.full((x.shape[0], 1), 11, dtype=torch.int64)
+    idx[:w.tokens] = exact_routes(STREAM_COUNTS, 7)[0]
+    idx, ones = idx.cuda(), torch.ones(x.shape[0], 1, device="cuda")
+
+    def run(a, b):
+        with torch.no_grad():
+            return m.run_direct_routed(x[a:b], ones[a:b], idx[a:b])
+
+    whole = run(0, x.shape[0])
+    assert torch.equal(whole[:w.tokens], run(0, w.tokens))
+    for step in (100, 300):
+        for a in range(w.tokens, x.shape[0], step):
+            assert torch.equal(whole[a:a + step], run(a, a + step))
