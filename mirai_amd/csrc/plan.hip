@@ -7,9 +7,11 @@
 // among the block's slots of the same expert is the popcount of the mask bits
 // below it, which is exactly the stable order of argsort(stable=True).
 // Pass 1 writes per-block expert counts (and per-block counts of invalid ids),
-// pass 2 (one workgroup) scans them into per-(block, expert) bases and writes
-// the plan's error count, pass 3 rebuilds the masks and scatters. Every
-// counter is written, not accumulated, so a plan needs no clearing launch.
+// pass 2 scans them into per-(block, expert) bases and writes the plan's error
+// count, pass 3 rebuilds the masks and scatters. Passes 2 and 3 are one kernel
+// up to 1024 experts and 32768 block counts, all three are one where a single
+// block takes the slots, and pass 2 is a launch of one workgroup otherwise.
+// Every counter is written, not accumulated, so a plan needs no clearing launch.
 #include "common.h"
 #include "plan.h"
 
@@ -278,6 +280,208 @@ __global__ __launch_bounds__(256) void plan_scatter_kernel(
   }
 }
 
+// Inclusive scan over a wave.
+__device__ __forceinline__ int32_t wave_scan(int32_t x) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1) {
+    const int32_t y = __shfl_up(x, off, 64);
+    x += lane >= off ? y : 0;
+  }
+  return x;
+}
+
+// Exclusive scans of N values per thread of a 1024-thread workgroup; `total`
+// receives the sums. `shared` holds 16 values per scan.
+template <int N>
+__device__ __forceinline__ void wg_exclusive_scan(const int32_t (&v)[N], int32_t (&before)[N],
+                                                  int32_t (&total)[N], int32_t *shared) {
+  const int lane = threadIdx.x & 63, wid = threadIdx.x >> 6;
+  int32_t x[N];
+#pragma unroll
+  for (int i = 0; i < N; ++i) x[i] = wave_scan(v[i]);
+  __syncthreads();  // the last use of `shared`
+  if (lane == 63) {
+#pragma unroll
+    for (int i = 0; i < N; ++i) shared[16 * i + wid] = x[i];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int i = 0; i < N; ++i) {
+    const int32_t s = wave_scan(lane < 16 ? shared[16 * i + lane] : 0);  // over the waves
+    const int32_t mine = __shfl(s, wid > 0 ? wid - 1 : 0, 64);
+    before[i] = (wid > 0 ? mine : 0) + x[i] - v[i];
+    total[i] = __shfl(s, 15, 64);
+  }
+}
+
+// The plan in one kernel after the block counts, or in one kernel altogether
+// when a single block holds every slot (n_blocks == 1, no counts passed).
+// Latency is all there is to it (a few hundred KB at most), so the scan is not
+// a launch of one workgroup between the counting and the scattering blocks:
+// every scattering block reads all the block counts itself (at most
+// kFusedCounts of them, from L2) and scans the experts, and one more block
+// writes the segments and the tile lists meanwhile. Kernel traces, 64 experts,
+// count + scan + scatter against this: 64 slots 19.4 -> 6.6 us and 1024 slots 15.4 ->
+// 9.7 (one launch for three), 16384 slots 23.1 -> 13.9, 131072 slots 24.8 -> 17.7;
+// 65536 slots of 128 experts 28.5 -> 23.0. (With 64-bit scans unrolled over the
+// waves the kernel spilled, and took 12.7 us for the 64 slots.)
+constexpr int kFusedCounts = 32768;
+// Mask bits (E * EB) of a block: masks and prefixes take 32 KB of LDS.
+constexpr int kFusedBits = 131072;
+
+struct PlanFused {
+  const int64_t *top_idx;
+  const void *top_scores;
+  int64_t R;
+  int k, E, EB, n_blocks;
+  const int32_t *block_counts, *block_err;
+  PlanView v;
+  int64_t *counts, *starts;
+  int32_t *offsets;
+  int64_t *sort_positions, *sorted_token_indices;
+  void *sorted_scores;
+  int64_t *inverse_order;
+};
+
+template <int SCORE_DTYPE>
+__global__ __launch_bounds__(1024) void plan_fused_kernel(PlanFused a) {
+  extern __shared__ uint32_t lds[];
+  __shared__ int32_t scan_tmp[64], part[1024], before_s[1024], base_s[1024];
+  __shared__ int32_t n_err;
+  const int t = threadIdx.x, E = a.E, words = a.EB >> 5;
+  const bool single = a.n_blocks == 1;
+  const int blk = blockIdx.x;
+  const bool scatters = blk < a.n_blocks, lists = blk == static_cast<int>(gridDim.x) - 1;
+  uint32_t *mask = lds, *prefix = lds + E * words;
+  const int64_t slot0 = static_cast<int64_t>(blk) * a.EB;
+  const int n_slots = static_cast<int>(min<int64_t>(a.EB, a.R - slot0));
+  if (t == 0) n_err = 0;
+  int32_t total = 0;  // rows of expert t
+  if (scatters) {
+    build_masks(a.top_idx, slot0, n_slots, E, words, mask, &n_err);
+    if (words <= 16) {
+      if (t < E) {
+        for (int w = 0; w < words; ++w) {
+          prefix[t * words + w] = total;
+          total += __popc(mask[t * words + w]);
+        }
+      }
+    } else {
+      for (int e = t >> 6; e < E; e += 16) {
+        int32_t run = 0;
+        for (int w0 = 0; w0 < words; w0 += 64) {
+          const int w = w0 + (t & 63);
+          const int32_t c = w < words ? __popc(mask[e * words + w]) : 0;
+          const int32_t x = wave_scan(c);
+          if (w < words) prefix[e * words + w] = run + x - c;
+          run += __shfl(x, 63, 64);
+        }
+        if ((t & 63) == 0) part[e] = run;
+      }
+      __syncthreads();
+      if (t < E) total = part[t];
+      __syncthreads();
+    }
+  }
+  int32_t before = 0;  // rows of expert t in the blocks before this one
+  if (!single) {
+    // Groups of E threads, each over a contiguous range of blocks.
+    const int G = max(1, min(16, 1024 / E)), g = t / E, e = t - g * E;
+    int32_t all = 0, mine = 0;
+    if (g < G) {
+      const int lo = a.n_blocks * g / G, hi = a.n_blocks * (g + 1) / G;
+#pragma unroll 8
+      for (int b = lo; b < hi; ++b) {
+        const int32_t c = a.block_counts[static_cast<int64_t>(b) * E + e];
+        all += c;
+        mine += b < blk ? c : 0;
+      }
+    }
+    __syncthreads();
+    part[t] = all;
+    before_s[t] = mine;
+    __syncthreads();
+    total = 0;
+    if (t < E)
+      for (int q = 0; q < G; ++q) {
+        total += part[q * E + t];
+        before += before_s[q * E + t];
+      }
+    if (lists) {
+      int32_t c = 0;
+      for (int b = t; b < a.n_blocks; b += 1024) c += a.block_err[b];
+      if (c) atomicAdd(&n_err, c);
+    }
+  }
+  int32_t start_[1], rows_[1];
+  wg_exclusive_scan<1>({total}, start_, rows_, scan_tmp);
+  const int32_t start = start_[0];
+  if (t < E) base_s[t] = start + before;
+  __syncthreads();
+  if (lists) {
+    if (t < E) {
+      a.v.seg[t] = start;
+      a.v.seg[E + t] = start + total;
+      if (a.counts) a.counts[t] = total;
+      if (a.starts) a.starts[t] = start;
+      if (a.offsets) a.offsets[t] = start + total;
+    }
+    // Tile counts of expert t in the four lists (as in plan_scan_kernel).
+    constexpr int M = kPlanTileM;
+    const int32_t full = total / (2 * M), rem = total - full * 2 * M;
+    const int32_t n[4] = {(total + M - 1) / M, full + (rem > 0 ? 1 : 0), full + (rem > M ? 1 : 0),
+                          rem > 0 && rem <= M ? 1 : 0};
+    int32_t at[4], num[4];
+    wg_exclusive_scan<4>(n, at, num, scan_tmp);
+    for (int j = 0; j < n[0]; ++j) a.v.tiles[at[0] + j] = make_int2(t, start + j * M);
+    for (int j = 0; j < n[1]; ++j) a.v.tiles2[at[1] + j] = make_int2(t, start + j * 2 * M);
+    for (int j = 0; j < n[2]; ++j) a.v.tiles2m[at[2] + j] = make_int2(t, start + j * 2 * M);
+    if (n[3]) a.v.tilesr[at[3]] = make_int2(t, start + full * 2 * M);
+    if (t == 0) {
+      *a.v.num_tiles = num[0];
+      *a.v.num_tiles2 = num[1];
+      *a.v.num_tiles2m = num[2];
+      *a.v.num_tilesr = num[3];
+      *a.v.err = n_err;
+    }
+  }
+  if (!scatters) return;
+  for (int p = t; p < n_slots; p += 1024) {
+    const int64_t i = slot0 + p;
+    const int64_t e = a.top_idx[i];
+    if (e < 0 || e >= E) {
+      if (a.inverse_order) a.inverse_order[i] = -1;
+      continue;
+    }
+    const int w = static_cast<int>(e) * words + (p >> 5);
+    const uint32_t below = mask[w] & ((1u << (p & 31)) - 1u);
+    const int32_t pos = base_s[e] + static_cast<int32_t>(prefix[w]) + __popc(below);
+    const uint32_t tok = static_cast<uint32_t>(i) / static_cast<uint32_t>(a.k);  // i < 2^31
+    if (a.sort_positions) a.sort_positions[pos] = i;
+    if (a.sorted_token_indices) a.sorted_token_indices[pos] = tok;
+    if (a.sorted_scores) {
+      if (SCORE_DTYPE == MX_DTYPE_BF16)
+        reinterpret_cast<uint16_t *>(a.sorted_scores)[pos] =
+            reinterpret_cast<const uint16_t *>(a.top_scores)[i];
+      else
+        reinterpret_cast<float *>(a.sorted_scores)[pos] =
+            reinterpret_cast<const float *>(a.top_scores)[i];
+    }
+    if (a.inverse_order) a.inverse_order[i] = pos;
+    a.v.row_token[pos] = static_cast<int32_t>(tok);
+    a.v.row_slot[pos] = static_cast<int32_t>(i);
+  }
+}
+
+// Slots per block when one block takes all R slots (a multiple of 32), or 0
+// when it cannot. 4096 slots take one workgroup about as long as a counting
+// launch of its own.
+inline int single_block_slots(int E, int64_t R) {
+  const int64_t eb = (R + 31) / 32 * 32;
+  return E <= 1024 && R <= 4096 && E * eb <= kFusedBits ? static_cast<int>(eb) : 0;
+}
+
 constexpr int kPlanMaxEpt = kPlanMaxExperts / 1024;
 
 }  // namespace
@@ -356,10 +560,41 @@ int build_plan(const int64_t *top_idx, const void *top_scores, int score_dtype,
   const int64_t R = num_tokens * top_k;
   const PlanLayout L = plan_layout(R, num_experts);
   const PlanView v = plan_view(workspace, L);
-  if (L.blocks > 0) {
+  const int eb1 = R > 0 ? single_block_slots(num_experts, R) : 0;
+  if (L.blocks > 0 && eb1 == 0) {
     const size_t lds = sizeof(uint32_t) * num_experts * (L.slots_per_block / 32);
     hipLaunchKernelGGL(plan_count_kernel, dim3(L.blocks), dim3(256), lds, s, top_idx, R,
                        num_experts, L.slots_per_block, v.block_counts, v.block_err);
+  }
+  // The fused kernel takes one expert per thread.
+  if (eb1 > 0 || (L.blocks > 1 && num_experts <= 1024 &&
+                  num_experts * L.slots_per_block <= kFusedBits &&
+                  static_cast<int64_t>(L.blocks) * num_experts <= kFusedCounts)) {
+    PlanFused a = {};
+    a.top_idx = top_idx;
+    a.top_scores = top_scores;
+    a.R = R;
+    a.k = top_k;
+    a.E = num_experts;
+    a.EB = eb1 > 0 ? eb1 : L.slots_per_block;
+    a.n_blocks = eb1 > 0 ? 1 : L.blocks;
+    a.block_counts = v.block_counts;
+    a.block_err = v.block_err;
+    a.v = v;
+    a.counts = counts;
+    a.starts = starts;
+    a.offsets = offsets;
+    a.sort_positions = sort_positions;
+    a.sorted_token_indices = sorted_token_indices;
+    a.sorted_scores = top_scores ? sorted_scores : nullptr;
+    a.inverse_order = inverse_order;
+    const size_t lds = 2 * sizeof(uint32_t) * num_experts * (a.EB / 32);
+    const dim3 grid(eb1 > 0 ? 1 : L.blocks + 1);
+    if (score_dtype == MX_DTYPE_BF16)
+      hipLaunchKernelGGL(plan_fused_kernel<MX_DTYPE_BF16>, grid, dim3(1024), lds, s, a);
+    else
+      hipLaunchKernelGGL(plan_fused_kernel<MX_DTYPE_F32>, grid, dim3(1024), lds, s, a);
+    return check_launch("mx_build_plan");
   }
   hipLaunchKernelGGL(num_experts <= 1024 ? plan_scan_kernel<1> : plan_scan_kernel<kPlanMaxEpt>,
                      dim3(1), dim3(1024), 0, s, v.block_counts,

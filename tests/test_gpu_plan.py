@@ -60,6 +60,28 @@ def test_plan_random_with_duplicates_and_invalid_ids(T, k, E):
     _check(idx, scores, E)
 
 
+@pytest.mark.parametrize("R,E", [
+    (1, 64), (31, 64), (33, 1), (2048, 64), (2049, 64), (4096, 32), (4097, 32), (128, 1024),
+    (129, 1024),              # one block, or just too many slots or mask bits for one
+    (65536, 128), (65537, 128),  # 256 blocks of 128 experts, and one more block
+    (20000, 1000), (3000, 65), (600, 2)])
+def test_plan_block_edges(R, E):
+    """Sizes on both sides of the rules that pick one block, fused or separate
+    scan kernels; skewed ids, invalid and dropped ones among them."""
+    from mirai_amd import _native as nat
+
+    rng = np.random.default_rng(R + E)
+    idx = np.minimum(rng.geometric(min(1.0, 8.0 / E), size=(R, 1)) - 1, E - 1).astype(np.int64)
+    scores = rng.standard_normal((R, 1)).astype(np.float32)
+    ids = idx.copy()
+    idx[3::50, 0] = E
+    ids[3::50, 0] = nat.ROUTE_DROPPED
+    plan = _check(idx, scores, E)
+    dropped = build_dispatch_plan(torch.from_numpy(ids).cuda(), torch.from_numpy(scores).cuda(), E)
+    for field in ("counts", "starts", "offsets", "inverse_order"):
+        assert torch.equal(getattr(plan, field), getattr(dropped, field))
+
+
 def test_plan_bf16_scores_and_zero_tokens():
     idx = np.zeros((0, 4), dtype=np.int64)
     plan = build_dispatch_plan(torch.from_numpy(idx).cuda(), torch.zeros((0, 4)).cuda(), 8)
