@@ -289,6 +289,11 @@ int mx_plan_from_counts(const int64_t *counts, int64_t num_rows, int num_experts
  * (device int32 pointer inside the workspace, for an optional host check). */
 const int32_t *mx_plan_error_counter(const void *workspace);
 
+/* Stores the plan error counter at the head of `workspace` into *host_slot, a
+ * mapped pinned host int32, on `stream` (a system-scope store: the host sees it
+ * without waiting for the stream). */
+int mx_publish_plan_errors(const void *workspace, int32_t *host_slot, void *stream);
+
 /* ------------------------------------------------------------------------ */
 /* Permute / combine                                                          */
 /* ------------------------------------------------------------------------ */

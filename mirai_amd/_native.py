@@ -140,6 +140,7 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
         c_int, [_P, _P, c_int, c_int64, c_int, c_int, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "mx_plan_from_counts": (c_int, [_P, c_int64, c_int, _P, _P]),
     "mx_plan_error_counter": (POINTER(c_int32), [_P]),
+    "mx_publish_plan_errors": (c_int, [_P, _P, _P]),
     "mx_gather_rows": (c_int, [_P, c_int64, _P, c_int64, c_int64, c_int, _P, _P]),
     "mx_scatter_add_rows": (c_int, [_P, _P, _P, c_int64, c_int64, c_int, c_int64, _P, _P]),
     "mx_combine": (c_int, [_P, _P, _P, c_int, c_int64, c_int, c_int, c_int64, _P, c_int, _P]),
@@ -263,7 +264,8 @@ def require_gpu(*tensors: torch.Tensor) -> torch.device:
 
 
 def stream(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+    """The current stream's raw handle (without building a torch Stream)."""
+    return torch._C._cuda_getCurrentRawStream(device.index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:
@@ -288,19 +290,21 @@ def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
 # into the workspace's error counter; such slots are left out of every
 # expert. The reference's torch.bincount raises on such ids
 # (dispatch_preprocess.py:155-157). Reading the counter needs the GPU to have
-# run the plan, so by default ("deferred") each call copies it into a pinned
-# host slot on its stream and the count is read once that copy has landed:
-# at the start of a later call, or by check_route_errors(), which waits. With
-# "sync" the call itself waits for its plan and raises; "off" skips the copy.
+# run the plan, so by default ("deferred") each call has it stored into a
+# pinned host slot on its stream (mx_publish_plan_errors) and the count is read
+# once it has landed (counts are not negative, an open slot holds -1): at the
+# start of a later call, or by check_route_errors(), which waits. With "sync"
+# the call itself waits for its plan and raises; "off" skips the store.
 # Calls captured into a HIP graph are not watched.
 ROUTE_CHECK_MODES = ("deferred", "sync", "off")
 _route_check = os.environ.get("MIRAI_ROUTE_CHECK", "deferred").strip().lower()
 if _route_check not in ROUTE_CHECK_MODES:  # pragma: no cover - environment
     _route_check = "deferred"
 _SLOTS = 256
-_slot_buf: torch.Tensor | None = None
+_slot_buf: torch.Tensor | None = None  # pinned int32 [_SLOTS]
+_slot_view: Any = None                 # the same memory as a ctypes array
 _slot_next = 0
-_pending: list = []  # (event, slot index, what)
+_pending: list = []  # (slot index, device, what)
 
 
 class RouteIndexError(ValueError):
@@ -331,14 +335,17 @@ def _raise_for(count: int, what: str, deferred: bool) -> None:
 
 def _drain(block: bool) -> None:
     while _pending:
-        event, slot, what = _pending[0]
-        if block:
-            event.synchronize()
-        elif not event.query():
-            return
+        slot, device, what = _pending[0]
+        if _slot_view[slot] < 0:
+            if not block:
+                return
+            torch.cuda.synchronize(device)
+        count = int(_slot_view[slot])
         _pending.pop(0)
-        count = int(_slot_buf[slot])
         if count:
+            # No store may still be on its way to a slot given out again.
+            for other in {d for _, d, _ in _pending}:
+                torch.cuda.synchronize(other)
             _pending.clear()
             _raise_for(count, what, deferred=True)
 
@@ -357,26 +364,26 @@ def check_route_errors() -> None:
 def watch_plan_errors(workspace: torch.Tensor, device: torch.device, what: str) -> None:
     """Queue the plan error counter at the head of ``workspace`` for reading
     (see ROUTE_CHECK_MODES); in "sync" mode wait for it and raise now."""
-    global _slot_buf, _slot_next
-    # Calls captured into a HIP graph are not watched: a capture may neither
-    # query events nor wait, and a replay would not refresh the slot.
+    global _slot_buf, _slot_view, _slot_next
+    # Calls captured into a HIP graph are not watched: a capture may not wait,
+    # and a replay would not refresh the slot.
     if _route_check == "off" or torch.cuda.is_current_stream_capturing():
         return
     if _slot_buf is None:
-        _slot_buf = torch.zeros(_SLOTS, dtype=torch.int32, pin_memory=True)
+        _slot_buf = torch.full((_SLOTS,), -1, dtype=torch.int32, pin_memory=True)
+        _slot_view = (c_int32 * _SLOTS).from_address(_slot_buf.data_ptr())
     slot = _slot_next
     _slot_next = (_slot_next + 1) % _SLOTS
-    # A slot is reused only after its previous copy has been read.
-    while any(p[1] == slot for p in _pending):
+    # A slot is reused only after its previous count has been read.
+    while len(_pending) >= _SLOTS:
         _drain(block=True)
-    counter = workspace[:4].view(torch.int32)
-    _slot_buf[slot:slot + 1].copy_(counter, non_blocking=True)
-    event = torch.cuda.Event()
-    event.record(torch.cuda.current_stream(device))
+    _slot_view[slot] = -1
+    call("mx_publish_plan_errors", workspace.data_ptr(), _slot_buf.data_ptr() + 4 * slot,
+         stream(device))
     if _route_check == "sync":
-        event.synchronize()
-        count = int(_slot_buf[slot])
+        torch.cuda.current_stream(device).synchronize()
+        count = int(_slot_view[slot])
         if count:
             _raise_for(count, what, deferred=False)
         return
-    _pending.append((event, slot, what))
+    _pending.append((slot, device, what))

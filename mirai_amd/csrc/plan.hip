@@ -695,6 +695,25 @@ extern "C" int mx_plan_from_counts(const int64_t *counts, int64_t num_rows, int 
   return plan_from_counts(counts, num_rows, num_experts, workspace, as_stream(stream));
 }
 
+namespace {
+__global__ void plan_publish_kernel(const int32_t *err, int32_t *host_slot) {
+  __hip_atomic_store(host_slot, *err, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+}  // namespace
+
+// One thread that stores the count through the mapped pointer: a 4-byte copy
+// to the host is a copy kernel of 4 us and an event of its own to wait for.
+extern "C" int mx_publish_plan_errors(const void *workspace, int32_t *host_slot, void *stream) {
+  clear_error();
+  if (!workspace || !host_slot) {
+    set_error("mx_publish_plan_errors: workspace and host slot must be non-null");
+    return MX_ERR_INVALID;
+  }
+  hipLaunchKernelGGL(plan_publish_kernel, dim3(1), dim3(1), 0, as_stream(stream),
+                     static_cast<const int32_t *>(workspace), host_slot);
+  return check_launch("mx_publish_plan_errors");
+}
+
 extern "C" const int32_t *mx_plan_error_counter(const void *workspace) {
   return static_cast<const int32_t *>(workspace);
 }

@@ -105,6 +105,8 @@ class CompressedGroupedExperts(nn.Module):
         self.num_experts = int(num_experts)
         self.mirai_expert_mlp_spec = execution_spec
         self._spec = spec
+        # Tensor names by role (gate, up, down), read on every call.
+        self._roles = tuple(spec.tensor_for_role(r) for r in ("gate", "up", "down"))
         self._group_sizes = group_sizes
         self._quant_format = quant.normalize_quant_format(quant_format)
         self._nf4_blocksize = int(nf4_blocksize)
@@ -327,11 +329,11 @@ class CompressedGroupedExperts(nn.Module):
                 f"compressed_weights grouped experts are missing weights: {missing}.")
 
     def _role_keys(self) -> tuple[str, str, str]:
-        return (self.projection_for_role("gate"), self.projection_for_role("up"),
-                self.projection_for_role("down"))
+        return self._roles
 
     def _adapters(self) -> list[ActiveExpertLoRA | None]:
-        return [self.expert_lora[k] if k in self.expert_lora else None for k in self._role_keys()]
+        attached = self.expert_lora._modules
+        return [attached.get(k) for k in self._roles]
 
     def run_direct_routed(self, tokens: torch.Tensor, top_scores: torch.Tensor,
                           top_indices: torch.Tensor) -> torch.Tensor:

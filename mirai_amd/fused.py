@@ -16,10 +16,11 @@ from . import _native as nat
 
 
 
-def lora_rank(module) -> int:
+def lora_rank(module, adapters=None) -> int:
     """Largest padded rank of the attached adapters (0 without LoRA): the
     ``lora_rank`` the native workspace queries are sized for."""
-    return max((a.padded_rank() for a in module._adapters() if a is not None), default=0)
+    adapters = module._adapters() if adapters is None else adapters
+    return max((a.padded_rank() for a in adapters if a is not None), default=0)
 
 
 def lora_row(module) -> int:
@@ -39,10 +40,10 @@ def kernel_activation(module) -> int:
     return act
 
 
-def _lora_descriptors(module, device, split=False):
+def _lora_descriptors(module, device, split=False, adapters=None):
     """MxLora structs for (gate, up, down) plus the bf16 factor tensors they point to."""
     descs, keep = [], []
-    for adapter in module._adapters():
+    for adapter in module._adapters() if adapters is None else adapters:
         if adapter is None:
             descs.append(nat.MxLora(None, None, 0, 0.0))
             continue
@@ -70,6 +71,13 @@ def _lora_params(module):
     return params
 
 
+def _needs_grad(module, *tensors) -> bool:
+    """Whether autograd has to see the call: a gradient can flow to one of the
+    tensors or to an adapter's factors."""
+    return torch.is_grad_enabled() and any(
+        t is not None and t.requires_grad for t in (*tensors, *_lora_params(module)))
+
+
 def _forward(module, tokens, top_scores, top_indices, need_grad, addend=None, addend_ready=None,
              out=None):
     """One mx_moe_forward call; returns (out, saved tensors or None). With an
@@ -92,7 +100,8 @@ def _forward(module, tokens, top_scores, top_indices, need_grad, addend=None, ad
     E = module.num_experts
     (w1, w3, w2), packed = _weight_descriptors(module, device)
     f = int(packed[0].shape[1])
-    lora, keep = _lora_descriptors(module, device, split)
+    adapters = module._adapters()
+    lora, keep = _lora_descriptors(module, device, split, adapters)
     out_dtype = tokens.dtype if tokens.dtype == torch.float32 else torch.bfloat16
     if out is None:
         out = torch.empty((T, d), dtype=out_dtype, device=device)
@@ -116,7 +125,8 @@ def _forward(module, tokens, top_scores, top_indices, need_grad, addend=None, ad
     if split:
         ws = nat.workspace(lib.mx_moe_f32x3_workspace_size(T, k, E, d, f), device)
     else:
-        ws = nat.workspace(lib.mx_moe_workspace_size(T, k, E, d, f, lora_rank(module)), device)
+        ws = nat.workspace(lib.mx_moe_workspace_size(T, k, E, d, f, lora_rank(module, adapters)),
+                           device)
     if addend is not None:
         if need_grad or split or addend.dtype != out.dtype or tuple(addend.shape) != (T, d):
             raise ValueError("the fused addend is a bf16 [tokens, hidden] inference input.")
@@ -250,9 +260,8 @@ class _Fp32RoutedExperts(torch.autograd.Function):
 def routed_experts(module, tokens, top_scores, top_indices):
     """The routed layer; with autograd only when a gradient can flow (in
     inference nothing is saved for a backward)."""
-    params = _lora_params(module)
-    if torch.is_grad_enabled() and any(
-            t is not None and t.requires_grad for t in (tokens, top_scores, *params)):
+    if _needs_grad(module, tokens, top_scores):
+        params = _lora_params(module)
         if module.quant_format == "fp32":
             return _Fp32RoutedExperts.apply(module, tokens, top_scores, top_indices, *params)
         return _RoutedExperts.apply(module, tokens, top_scores, top_indices, *params)
@@ -319,9 +328,8 @@ def routed_experts_chunked(module, tokens, top_scores, top_indices, bounds):
     bounds = [(int(a), int(b)) for a, b in bounds if int(b) > int(a)]
     if not bounds:
         return routed_experts(module, tokens, top_scores, top_indices)
-    params = _lora_params(module)
-    if torch.is_grad_enabled() and any(
-            t is not None and t.requires_grad for t in (tokens, top_scores, *params)):
+    if _needs_grad(module, tokens, top_scores):
+        params = _lora_params(module)
         if module.quant_format == "fp32":
             # Each chunk's backward recomputes only that chunk's fp32 layer.
             return torch.cat([
@@ -337,9 +345,7 @@ def routed_experts_chunked(module, tokens, top_scores, top_indices, bounds):
 def routed_experts_plus(module, tokens, top_scores, top_indices, addend, addend_ready=None):
     """routed_experts(...) + addend, the add fused into the combine in inference
     (the combine waits for ``addend_ready``); with autograd a plain add."""
-    params = _lora_params(module)
-    if torch.is_grad_enabled() and any(
-            t is not None and t.requires_grad for t in (tokens, top_scores, addend, *params)):
+    if _needs_grad(module, tokens, top_scores, addend):
         if addend_ready is not None:
             torch.cuda.current_stream(tokens.device).wait_event(addend_ready)
         return routed_experts(module, tokens, top_scores, top_indices) + addend
@@ -492,10 +498,8 @@ def expert_choice_experts(module, tokens, expert_token_scores, expert_token_indi
     """Expert-choice routed layer through mx_moe_forward_expert_choice_ex; with
     autograd (gradients to tokens, scores and the LoRA factors) when one of
     them requires a gradient."""
-    params = _lora_params(module)
-    if torch.is_grad_enabled() and any(
-            t is not None and t.requires_grad
-            for t in (tokens, expert_token_scores, *params)):
+    if _needs_grad(module, tokens, expert_token_scores):
+        params = _lora_params(module)
         _ec_inputs(module, tokens, expert_token_scores, expert_token_indices, tokens_per_sample,
                    aliases)  # validates before autograd records anything
         return _ExpertChoiceExperts.apply(module, int(tokens_per_sample), tuple(aliases), tokens,
@@ -520,8 +524,7 @@ def sorted_experts(module, tokens, counts):
             raise ValueError(f"counts sum to {int(idx.numel())}, but {S} rows were given.")
         ones = torch.ones((S, 1), dtype=torch.float32, device=device)
         return routed_experts(module, tokens, ones, idx.view(S, 1))
-    if torch.is_grad_enabled() and (tokens.requires_grad or any(
-            p is not None and p.requires_grad for p in _lora_params(module))):
+    if _needs_grad(module, tokens):
         from .backward import sorted_experts_autograd
         return sorted_experts_autograd(module, tokens, counts)
     x = tokens.detach().to(torch.bfloat16).contiguous()

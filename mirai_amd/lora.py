@@ -73,7 +73,7 @@ class ActiveExpertLoRA(nn.Module):
         the buffer changes: a read per call would synchronise the host with the
         GPU on every forward, and cannot happen under HIP graph capture."""
         buf = self.lora_alpha
-        key = (buf.data_ptr(), buf._version, str(buf.device))
+        key = (buf.data_ptr(), buf._version, buf.device)
         cached = self.__dict__.get("_alpha_cache")
         if cached is None or cached[0] != key:
             cached = (key, float(buf))
@@ -101,8 +101,8 @@ class ActiveExpertLoRA(nn.Module):
         """
         # The packed copies are kept while the parameters are unchanged (same
         # storage, same in-place version), so inference packs them once.
-        key = (str(device), bool(split), self.lora_a.data_ptr(), self.lora_a._version,
-               self.lora_b.data_ptr(), self.lora_b._version)
+        a, b = self.lora_a, self.lora_b
+        key = (device, bool(split), a.data_ptr(), a._version, b.data_ptr(), b._version)
         cached = self.__dict__.get("_kernel_cache")
         if cached is not None and cached[0] == key:
             return cached[1]
