@@ -9,7 +9,7 @@
 // Pass 1 writes per-block expert counts (and per-block counts of invalid ids),
 // pass 2 scans them into per-(block, expert) bases and writes the plan's error
 // count, pass 3 rebuilds the masks and scatters. Passes 2 and 3 are one kernel
-// up to 1024 experts and 32768 block counts, all three are one where a single
+// up to 1024 experts and 65536 block counts, all three are one where a single
 // block takes the slots, and pass 2 is a launch of one workgroup otherwise.
 // Every counter is written, not accumulated, so a plan needs no clearing launch.
 #include "common.h"
@@ -324,9 +324,11 @@ __device__ __forceinline__ void wg_exclusive_scan(const int32_t (&v)[N], int32_t
 // writes the segments and the tile lists meanwhile. Kernel traces, 64 experts,
 // count + scan + scatter against this: 64 slots 19.4 -> 6.6 us and 1024 slots 15.4 ->
 // 9.7 (one launch for three), 16384 slots 23.1 -> 13.9, 131072 slots 24.8 -> 17.7;
-// 65536 slots of 128 experts 28.5 -> 23.0. (With 64-bit scans unrolled over the
+// 65536 slots of 128 experts 28.5 -> 23.0. Kernel times alone, without the gaps between
+// them, 256 experts: 38400 slots 26.0 -> 14.0, 65536 slots (65536 block counts, the
+// most) 30.4 -> 20.7; 98304 slots of 128 experts 27.8 -> 18.8. (With 64-bit scans unrolled over the
 // waves the kernel spilled, and took 12.7 us for the 64 slots.)
-constexpr int kFusedCounts = 32768;
+constexpr int kFusedCounts = 65536;
 // Mask bits (E * EB) of a block: masks and prefixes take 32 KB of LDS.
 constexpr int kFusedBits = 131072;
 

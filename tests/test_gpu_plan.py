@@ -64,6 +64,7 @@ def test_plan_random_with_duplicates_and_invalid_ids(T, k, E):
     (1, 64), (31, 64), (33, 1), (2048, 64), (2049, 64), (4096, 32), (4097, 32), (128, 1024),
     (129, 1024),              # one block, or just too many slots or mask bits for one
     (65536, 128), (65537, 128),  # 256 blocks of 128 experts, and one more block
+    (65536, 256), (65537, 256),  # 65536 block counts, and 256 more
     (20000, 1000), (3000, 65), (600, 2)])
 def test_plan_block_edges(R, E):
     """Sizes on both sides of the rules that pick one block, fused or separate
