@@ -559,6 +559,21 @@ int mx_moe_forward_ex(const void *tokens, const int64_t *top_idx, const void *to
                       void *stream);
 
 /*
+ * mx_moe_forward_ex whose plan also stores its error count into *host_slot, a
+ * mapped pinned host int32 (NULL: mx_moe_forward_ex), with a system-scope
+ * store: the host sees it without waiting for the stream. A call with no tokens
+ * builds no plan and stores nothing.
+ */
+int mx_moe_forward_watched(const void *tokens, const int64_t *top_idx, const void *top_scores,
+                           int score_dtype, int64_t num_tokens, int top_k, int num_experts,
+                           int64_t hidden, int64_t ffn, int act, const mx_weight *w1,
+                           const mx_weight *w3, const mx_weight *w2, const mx_lora *l1,
+                           const mx_lora *l3, const mx_lora *l2, void *out, int out_dtype,
+                           const void *addend, void *addend_ready, void *save_gate,
+                           void *save_up, void *save_h, void *save_y, void *save_lora,
+                           void *workspace, int32_t *host_slot, void *stream);
+
+/*
  * Expert-choice routes: expert_token_indices / expert_token_scores [B, L, C]
  * (each of L logical experts picks C tokens of each of B samples; token ids
  * in [0, tokens_per_sample)). The flat slots s = (b, l, c) map to physical

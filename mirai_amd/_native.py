@@ -170,6 +170,10 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
         c_int,
         [_P, _P, _P, c_int, c_int64, c_int, c_int, c_int64, c_int64, c_int, _W, _W, _W, _L, _L,
          _L, _P, c_int, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
+    "mx_moe_forward_watched": (
+        c_int,
+        [_P, _P, _P, c_int, c_int64, c_int, c_int, c_int64, c_int64, c_int, _W, _W, _W, _L, _L,
+         _L, _P, c_int, _P, _P, _P, _P, _P, _P, _P, _P, _P, _P]),
     "mx_moe_forward_static": (
         c_int,
         [_P, _P, _P, c_int, c_int64, c_int, c_int, c_int64, c_int64, c_int, _W, _W, _W, _L, _L,
@@ -291,8 +295,8 @@ def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
 # expert. The reference's torch.bincount raises on such ids
 # (dispatch_preprocess.py:155-157). Reading the counter needs the GPU to have
 # run the plan, so by default ("deferred") each call has it stored into a
-# pinned host slot on its stream (mx_publish_plan_errors) and the count is read
-# once it has landed (counts are not negative, an open slot holds -1): at the
+# pinned host slot on its stream (by the layer's plan, or mx_publish_plan_errors)
+# and the count is read once it has landed (counts are not negative, an open slot holds -1): at the
 # start of a later call, or by check_route_errors(), which waits. With "sync"
 # the call itself waits for its plan and raises; "off" skips the store.
 # Calls captured into a HIP graph are not watched.
@@ -361,25 +365,33 @@ def check_route_errors() -> None:
     _drain(block=True)
 
 
-def watch_plan_errors(workspace: torch.Tensor, device: torch.device, what: str) -> None:
-    """Queue the plan error counter at the head of ``workspace`` for reading
-    (see ROUTE_CHECK_MODES); in "sync" mode wait for it and raise now."""
+def open_error_slot() -> tuple[int, int] | None:
+    """A pinned slot (index, address) for a call's plan error count, or None
+    where calls are not watched. watch_error_slot follows once the launch that
+    fills it is queued."""
     global _slot_buf, _slot_view, _slot_next
     # Calls captured into a HIP graph are not watched: a capture may not wait,
     # and a replay would not refresh the slot.
     if _route_check == "off" or torch.cuda.is_current_stream_capturing():
-        return
+        return None
     if _slot_buf is None:
         _slot_buf = torch.full((_SLOTS,), -1, dtype=torch.int32, pin_memory=True)
         _slot_view = (c_int32 * _SLOTS).from_address(_slot_buf.data_ptr())
     slot = _slot_next
     _slot_next = (_slot_next + 1) % _SLOTS
     # A slot is reused only after its previous count has been read.
-    while len(_pending) >= _SLOTS:
+    while any(p[0] == slot for p in _pending):
         _drain(block=True)
     _slot_view[slot] = -1
-    call("mx_publish_plan_errors", workspace.data_ptr(), _slot_buf.data_ptr() + 4 * slot,
-         stream(device))
+    return slot, _slot_buf.data_ptr() + 4 * slot
+
+
+def watch_error_slot(opened: tuple[int, int] | None, device: torch.device, what: str) -> None:
+    """Queue an opened slot for reading (see ROUTE_CHECK_MODES); in "sync" mode
+    wait for its count and raise now."""
+    if opened is None:
+        return
+    slot = opened[0]
     if _route_check == "sync":
         torch.cuda.current_stream(device).synchronize()
         count = int(_slot_view[slot])
@@ -387,3 +399,12 @@ def watch_plan_errors(workspace: torch.Tensor, device: torch.device, what: str) 
             _raise_for(count, what, deferred=False)
         return
     _pending.append((slot, device, what))
+
+
+def watch_plan_errors(workspace: torch.Tensor, device: torch.device, what: str) -> None:
+    """Watch the plan error counter at the head of ``workspace``, stored into a
+    slot by a launch of its own."""
+    opened = open_error_slot()
+    if opened is not None:
+        call("mx_publish_plan_errors", workspace.data_ptr(), opened[1], stream(device))
+        watch_error_slot(opened, device, what)

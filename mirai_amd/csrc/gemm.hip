@@ -2787,15 +2787,13 @@ extern "C" size_t mx_moe_f32x3_workspace_size(int64_t num_tokens, int top_k, int
   return layer_layout(num_tokens * top_k, num_experts, hidden, ffn, true, num_tokens).bytes;
 }
 
-extern "C" int mx_moe_forward_ex(const void *tokens, const int64_t *top_idx,
-                                 const void *top_scores, int score_dtype, int64_t num_tokens,
-                                 int top_k, int num_experts, int64_t hidden, int64_t ffn, int act,
-                                 const mx_weight *w1, const mx_weight *w3, const mx_weight *w2,
-                                 const mx_lora *l1, const mx_lora *l3, const mx_lora *l2,
-                                 void *out, int out_dtype, const void *addend,
-                                 void *addend_ready, void *save_gate, void *save_up,
-                                 void *save_h, void *save_y, void *save_lora, void *workspace,
-                                 void *stream) {
+extern "C" int mx_moe_forward_watched(
+    const void *tokens, const int64_t *top_idx, const void *top_scores, int score_dtype,
+    int64_t num_tokens, int top_k, int num_experts, int64_t hidden, int64_t ffn, int act,
+    const mx_weight *w1, const mx_weight *w3, const mx_weight *w2, const mx_lora *l1,
+    const mx_lora *l3, const mx_lora *l2, void *out, int out_dtype, const void *addend,
+    void *addend_ready, void *save_gate, void *save_up, void *save_h, void *save_y,
+    void *save_lora, void *workspace, int32_t *host_slot, void *stream) {
   clear_error();
   const char *name = "mx_moe_forward";
   int rc = validate_plan_args(name, num_tokens, top_k, num_experts);
@@ -2843,7 +2841,7 @@ extern "C" int mx_moe_forward_ex(const void *tokens, const int64_t *top_idx,
     x = xs;
   }
   rc = build_plan(top_idx, nullptr, score_dtype, num_tokens, top_k, num_experts, nullptr, nullptr,
-                  nullptr, nullptr, nullptr, nullptr, nullptr, ws, s);
+                  nullptr, nullptr, nullptr, nullptr, nullptr, ws, s, host_slot);
   if (rc) return rc;
   mark_stage(1, s);
   uint16_t *lora_buf = save_lora ? static_cast<uint16_t *>(save_lora)
@@ -2878,6 +2876,21 @@ extern "C" int mx_moe_forward_ex(const void *tokens, const int64_t *top_idx,
   }
   mark_stage(6, s);
   return rc;
+}
+
+extern "C" int mx_moe_forward_ex(const void *tokens, const int64_t *top_idx,
+                                 const void *top_scores, int score_dtype, int64_t num_tokens,
+                                 int top_k, int num_experts, int64_t hidden, int64_t ffn, int act,
+                                 const mx_weight *w1, const mx_weight *w3, const mx_weight *w2,
+                                 const mx_lora *l1, const mx_lora *l3, const mx_lora *l2,
+                                 void *out, int out_dtype, const void *addend,
+                                 void *addend_ready, void *save_gate, void *save_up,
+                                 void *save_h, void *save_y, void *save_lora, void *workspace,
+                                 void *stream) {
+  return mx_moe_forward_watched(tokens, top_idx, top_scores, score_dtype, num_tokens, top_k,
+                                num_experts, hidden, ffn, act, w1, w3, w2, l1, l3, l2, out,
+                                out_dtype, addend, addend_ready, save_gate, save_up, save_h,
+                                save_y, save_lora, workspace, nullptr, stream);
 }
 
 extern "C" int mx_moe_forward_act(const void *tokens, const int64_t *top_idx,

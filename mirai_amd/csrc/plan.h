@@ -58,10 +58,13 @@ PlanLayout plan_layout(int64_t num_rows, int num_experts);
 PlanView plan_view(void *ws, const PlanLayout &L);
 int validate_plan_args(const char *name, int64_t num_tokens, int top_k, int num_experts);
 
+// host_err (mapped pinned host memory, or null) receives the error count too, as
+// soon as it is known.
 int build_plan(const int64_t *top_idx, const void *top_scores, int score_dtype,
                int64_t num_tokens, int top_k, int num_experts, int64_t *counts, int64_t *starts,
                int32_t *offsets, int64_t *sort_positions, int64_t *sorted_token_indices,
-               void *sorted_scores, int64_t *inverse_order, void *workspace, hipStream_t s);
+               void *sorted_scores, int64_t *inverse_order, void *workspace, hipStream_t s,
+               int32_t *host_err = nullptr);
 int plan_from_counts(const int64_t *counts, int64_t num_rows, int num_experts, void *workspace,
                      hipStream_t s);
 

@@ -79,6 +79,15 @@ __device__ int64_t block_exclusive_scan(int64_t v, int64_t *shared, int64_t *tot
   return r;
 }
 
+// The plan's error count, and its copy for the host (system scope: the host
+// sees it while the stream is still busy). As a launch of its own after the
+// layer this store took 4 us, and as long as the last workgroup slot took to
+// come free beside another stream's work (14 us beside a GEMM).
+__device__ __forceinline__ void store_errors(int32_t n, int32_t *err, int32_t *host_err) {
+  *err = n;
+  if (host_err) __hip_atomic_store(host_err, n, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // One workgroup of 1024 threads. Thread t owns experts t, t + 1024, ...
 // (E <= kPlanMaxExperts); the exclusive scans over experts run chunk by chunk
 // of 1024 in expert order, carrying the running total. With E <= 1024 the
@@ -91,7 +100,8 @@ __global__ __launch_bounds__(1024) void plan_scan_kernel(
     const int32_t *block_counts, const int32_t *block_err, int n_blocks, int E, int64_t n_rows,
     int tile_m, const int64_t *counts_in, int32_t *block_base, int64_t *seg, int2 *tiles,
     int32_t *num_tiles, int2 *tiles2, int32_t *num_tiles2, int2 *tiles2m, int32_t *num_tiles2m,
-    int2 *tilesr, int32_t *num_tilesr, int32_t *err_counter, int64_t *counts_out,
+    int2 *tilesr, int32_t *num_tilesr, int32_t *err_counter, int32_t *host_err,
+    int64_t *counts_out,
     int64_t *starts_out, int32_t *offsets_out) {
   __shared__ int64_t scan_tmp[32];
   __shared__ int32_t part[1024];     // [group][expert] block-range counts (E <= 1024)
@@ -218,7 +228,7 @@ __global__ __launch_bounds__(1024) void plan_scan_kernel(
     }
   }
   __syncthreads();
-  if (t == 0) *err_counter = n_err;
+  if (t == 0) store_errors(n_err, err_counter, host_err);
 }
 
 template <int SCORE_DTYPE>
@@ -339,6 +349,7 @@ struct PlanFused {
   int k, E, EB, n_blocks;
   const int32_t *block_counts, *block_err;
   PlanView v;
+  int32_t *host_err;
   int64_t *counts, *starts;
   int32_t *offsets;
   int64_t *sort_positions, *sorted_token_indices;
@@ -445,7 +456,7 @@ __global__ __launch_bounds__(1024) void plan_fused_kernel(PlanFused a) {
       *a.v.num_tiles2 = num[1];
       *a.v.num_tiles2m = num[2];
       *a.v.num_tilesr = num[3];
-      *a.v.err = n_err;
+      store_errors(n_err, a.v.err, a.host_err);
     }
   }
   if (!scatters) return;
@@ -558,7 +569,8 @@ PlanView plan_view(void *ws, const PlanLayout &L) {
 int build_plan(const int64_t *top_idx, const void *top_scores, int score_dtype,
                int64_t num_tokens, int top_k, int num_experts, int64_t *counts, int64_t *starts,
                int32_t *offsets, int64_t *sort_positions, int64_t *sorted_token_indices,
-               void *sorted_scores, int64_t *inverse_order, void *workspace, hipStream_t s) {
+               void *sorted_scores, int64_t *inverse_order, void *workspace, hipStream_t s,
+               int32_t *host_err) {
   const int64_t R = num_tokens * top_k;
   const PlanLayout L = plan_layout(R, num_experts);
   const PlanView v = plan_view(workspace, L);
@@ -583,6 +595,7 @@ int build_plan(const int64_t *top_idx, const void *top_scores, int score_dtype,
     a.block_counts = v.block_counts;
     a.block_err = v.block_err;
     a.v = v;
+    a.host_err = host_err;
     a.counts = counts;
     a.starts = starts;
     a.offsets = offsets;
@@ -604,7 +617,7 @@ int build_plan(const int64_t *top_idx, const void *top_scores, int score_dtype,
                      num_experts, R,
                      kPlanTileM, static_cast<const int64_t *>(nullptr), v.block_base, v.seg,
                      v.tiles, v.num_tiles, v.tiles2, v.num_tiles2, v.tiles2m, v.num_tiles2m,
-                     v.tilesr, v.num_tilesr, v.err, counts, starts, offsets);
+                     v.tilesr, v.num_tilesr, v.err, host_err, counts, starts, offsets);
   if (L.blocks > 0) {
     const size_t lds = (plan_prefix_in_lds(num_experts, L.slots_per_block) ? 2 : 1) *
                        sizeof(uint32_t) * num_experts * (L.slots_per_block / 32);
@@ -634,7 +647,8 @@ int plan_from_counts(const int64_t *counts, int64_t num_rows, int num_experts, v
                      0, num_experts, num_rows,
                      kPlanTileM, counts, static_cast<int32_t *>(nullptr), v.seg, v.tiles,
                      v.num_tiles, v.tiles2, v.num_tiles2, v.tiles2m, v.num_tiles2m, v.tilesr,
-                     v.num_tilesr, v.err, static_cast<int64_t *>(nullptr),
+                     v.num_tilesr, v.err, static_cast<int32_t *>(nullptr),
+                     static_cast<int64_t *>(nullptr),
                      static_cast<int64_t *>(nullptr), static_cast<int32_t *>(nullptr));
   return check_launch("mx_plan_from_counts");
 }
