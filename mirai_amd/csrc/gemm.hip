@@ -2566,8 +2566,13 @@ int backward_core(const BackLayout &L, const PlanView &v, int num_experts, int64
     const int r = l2->rank;
     const mx_lora t = {fact[0], nullptr, r, l2->scale};
     const mx_lora *ad[1] = {&t};
+    // Few tiles run in K parts as the forward's (one workgroup per tile walked K
+    // alone: 8184 rows of 128 experts, rank 64, K 2048, 33 us; now 20 and 5 for the
+    // finishing pass), with their sums in [dG | dU], which the dh GEMM writes next.
+    // The dz passes over [dG | dU] have no buffer free and a short K.
     if ((rc = lora_down(v, num_experts, L.plan.max_tiles, dy, hidden, v.row_slot, hidden, ad, 1,
-                        lrc, dz + 2 * lrc, ldz, s)))
+                        lrc, dz + 2 * lrc, ldz, s, false, R, reinterpret_cast<float *>(dgu),
+                        sizeof(uint16_t) * R * 2 * ffn)))
       return rc;
   }
   mark_stage(2, s);

@@ -121,6 +121,14 @@ def test_backward_lora_ranks(r):
     _case(small("nf4", r=r, alpha=2.0 * r, E=5, k=3, T=300, f=320, d=192))
 
 
+@pytest.mark.parametrize("d,f,r", [(1024, 192, 16), (2048, 320, 64), (2048, 192, 64),
+                                   (1088, 320, 16)])
+def test_backward_lora_sums_in_k_parts(d, f, r):
+    # dz2's K sum (over d) in 2 and 4 parts of their own workgroups; not split where
+    # [dG | dU] is too small for the parts' sums, nor at 17 K steps.
+    _case(small("nf4", T=100, d=d, f=f, E=4, r=r))
+
+
 def test_backward_mixed_lora_ranks_on_tall_tiles():
     w = small("int8", E=4, k=2, T=1100, f=256, d=192, alpha=32.0)
     _case(w, lora=mixed_rank_factors(w, {"w1": 96, "w3": 24, "w2": 64}))
