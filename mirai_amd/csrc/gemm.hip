@@ -1317,10 +1317,15 @@ constexpr int stream_kstep() {
   return FMT == MX_FMT_BF16 ? 64 : 128;
 }
 
-template <int FMT, int EPI, bool LORA, int MB>
+// BLOCKWISE (NF4, one row block): each half-wave multiplies its own 64-block of
+// a step, MFMA step s taking its columns 8 s .. + 7 for weights and tokens
+// alike: no exchange between the halves, and another order of the sum over K
+// than that of all other tiles.
+template <int FMT, int EPI, bool LORA, int MB, bool BLOCKWISE = false>
 __device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, uint8_t *sA0,
                                             uint8_t *sA1, const float *sCode) {
   constexpr int KS = stream_kstep<FMT>();
+  static_assert(!BLOCKWISE || (is_nf4(FMT) && MB == 1), "blockwise order: NF4, 32 rows");
   constexpr int SUB = KS / 16;          // MFMA steps per K step
   constexpr int kRowsPerDma = 512 / KS; // token rows one DMA instruction fills
   constexpr int kDmas = MB * 32 / kRowsPerDma;
@@ -1419,8 +1424,10 @@ __device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, 
 
   // The lane's fragment of MFMA step s in row block 0: chunk 2 s + h of row
   // li, at frag0 ^ (s << 5) (h has no bit of 2 s; blocks of 32 rows repeat the
-  // row key).
-  int frag0 = li * (2 * KS) + ((h ^ (KS == 64 ? swz_key64(li) : (li & 15))) << 4);
+  // row key). Blockwise: chunk s + 8 h, at frag0 ^ (s << 4).
+  constexpr int kFragShift = BLOCKWISE ? 4 : 5;
+  int frag0 = li * (2 * KS) +
+              (((BLOCKWISE ? 8 * h : h) ^ (KS == 64 ? swz_key64(li) : (li & 15))) << 4);
   // One K step on stage `cur`: the barrier publishes its rows (loaded during
   // the step before) and frees the other stage, whose next rows and the next
   // codes then load while this step multiplies.
@@ -1437,9 +1444,9 @@ __device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, 
     // (one XOR each) instead of held in registers over the loop.
     asm volatile("" : "+v"(frag0));
     // The step's 128 K columns are two 64-blocks of the row, block h loaded by
-    // half h. The MFMA takes K in natural order (half h: columns 16 s + 8 h ..
-    // + 7, as every other tile, so a row's sum has the same bits whichever
-    // tile runs it): the halves swap every second group of 8, after which both
+    // half h. Unless BLOCKWISE the MFMA takes K in natural order (half h: columns
+    // 16 s + 8 h .. + 7, as the tiles that stage decoded weights, so that a row's
+    // sum has their bits): the halves swap every second group of 8, after which both
     // hold their columns of block 0 in the even groups and of block 1 in the
     // odd ones. Of the NF4 blocks either the decode tables are swapped likewise
     // (t0, t1), or, where the accumulators leave no registers for two tables,
@@ -1451,7 +1458,7 @@ __device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, 
 #pragma unroll
     for (int q = 0; q < 4 * kQ; ++q) w[q] = cc.q[q >> 2][q & 3];
     float abs0 = 0.0f, abs1 = 0.0f;
-    if constexpr (KS == 128) {
+    if constexpr (KS == 128 && !BLOCKWISE) {
 #pragma unroll
       for (int g = 0; g < 8; g += 2)
 #pragma unroll
@@ -1464,7 +1471,9 @@ __device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, 
         av = dq_absmax(sCode[which * 256 + cc.abs], 2 * b + h < dq_sw ? dq_lo : dq_hi, dq_off);
       else
         av = absmax_value<FMT>(cc.abs);
-      if constexpr (kSwapTables) {
+      if constexpr (BLOCKWISE) {
+        t0 = nf4_table(av);
+      } else if constexpr (kSwapTables) {
         t0 = t1 = nf4_table(av);
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -1483,16 +1492,16 @@ __device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, 
     for (int s = 0; s < SUB; ++s) {
       if constexpr (is_nf4(FMT)) {
         if (kSwapTables)
-          t = s < SUB / 2 ? t0 : t1;
+          t = BLOCKWISE || s < SUB / 2 ? t0 : t1;
         else if (s % (SUB / 2) == 0)
           t = nf4_table(s == 0 ? abs0 : abs1);
       }
       bf16x8 a[MB];
 #pragma unroll
       for (int mb = 0; mb < MB; ++mb)
-        a[mb] = *reinterpret_cast<const bf16x8 *>(cur + (frag0 ^ (s << 5)) + 32 * mb * (2 * KS));
+        a[mb] = *reinterpret_cast<const bf16x8 *>(cur + (frag0 ^ (s << kFragShift)) + 32 * mb * (2 * KS));
       // Group of MFMA step s: the even ones of block 0, then the odd ones.
-      const int g = 2 * (s & 3) + (s >> 2);
+      const int g = BLOCKWISE ? s : 2 * (s & 3) + (s >> 2);
       uint32_t d[4];
       if constexpr (is_nf4(FMT)) {
         nf4_decode8(t, w[g], d);
@@ -1598,11 +1607,20 @@ __device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, 
   }
 }
 
-// The tile's rows in the fewest row blocks.
+// The tile's rows in the fewest row blocks. NF4 tiles of at most 32 rows sum K
+// blockwise up to kBlockwiseK columns: the order, and so the bits, that rows of
+// such experts have always had.
+constexpr int kBlockwiseK = 2048;
 template <int FMT, int EPI, bool LORA>
 __device__ __forceinline__ void stream_rows(const Params &p, int2 tile, int nt, uint8_t *sA0,
                                             uint8_t *sA1, const float *sCode) {
   const int64_t m = p.seg_end[tile.x] - tile.y;
+  if constexpr (is_nf4(FMT)) {
+    if (m <= 32 && p.K <= kBlockwiseK) {
+      stream_tile<FMT, EPI, LORA, 1, true>(p, tile, nt, sA0, sA1, sCode);
+      return;
+    }
+  }
   if (m <= 32)
     stream_tile<FMT, EPI, LORA, 1>(p, tile, nt, sA0, sA1, sCode);
   else if (m <= 64)

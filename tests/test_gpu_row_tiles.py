@@ -13,6 +13,7 @@ import pytest
 import torch
 
 from mirai_amd import workloads as wl
+from oracle import codec
 from oracle import layer as olayer
 
 from helpers import assert_layer_close, build_module, oracle_loras, oracle_weights
@@ -97,7 +98,8 @@ def test_streaming_tiles(fmt, d, f, rank):
 def test_a_rows_bits_do_not_depend_on_the_launch(fmt):
     # The same rows of experts 0 .. 10 alone (streaming launch) and beside a
     # heavy expert 11 (the launch with 256-row tiles), and the heavy expert's
-    # rows in 300s (256 + 44) and in 100s: every tile sums K in one order.
+    # rows in 300s (256 + 44) and in 100s: tiles of more than 32 rows sum K in one
+    # order, smaller ones in theirs in either launch.
     w = workload(fmt, STREAM_COUNTS, d=640, f=384)
     m = build_module(w, wl.dense_weights(w), wl.lora_factors(w))
     x = wl.tokens(w.with_tokens(w.tokens + 900)).cuda()
@@ -114,3 +116,50 @@ def test_a_rows_bits_do_not_depend_on_the_launch(fmt):
     for step in (100, 300):
         for a in range(w.tokens, x.shape[0], step):
             assert torch.equal(whole[a:a + step], run(a, a + step))
+
+
+def _blockwise(K):
+    """Positions of the columns 64 h + 8 s + j of each 128-block after the order
+    16 s + 8 h + j."""
+    k = torch.arange(K).view(K // 128, 2, 8, 8)
+    return k.permute(0, 2, 1, 3).reshape(K)
+
+
+@pytest.mark.parametrize("heavy", [0, 300])
+@pytest.mark.parametrize("m", [1, 31, 32])
+@pytest.mark.parametrize("d,f", [(256, 384), (640, 768), (2048, 640), (2176, 640)])
+def test_few_rows_sum_k_blockwise(d, f, m, heavy):
+    """NF4 tiles of at most 32 rows and 2048 columns of K sum K as half-waves
+    read it (columns 8 s .. + 7 of both 64-blocks of a step together); tiles of
+    more rows or columns take 16 columns in a row. So m rows alone give the
+    bits that they give beside another 33 rows of their expert once K's
+    columns are reordered; every block has one absmax, so reordering does not
+    change what the weights stand for. ``heavy`` rows of the other expert bring
+    the launch with 256-row tiles (K above 512) or leave it out."""
+    g = torch.Generator().manual_seed(31 * d + m)
+    w = wl.Workload("blockwise", 13, m, d, f, 2, 1, 1, 1.0, "nf4", torch.bfloat16)
+    levels = torch.from_numpy(codec.NF4_LEVELS).to(torch.bfloat16)
+
+    def weight(o, i):
+        t = levels[torch.randint(0, 16, (2, o, i), generator=g)]
+        t[:, :, ::8] = 1.0  # every 64-block's absmax, before and after the reordering
+        return t / 32
+
+    dense = {"w1": weight(f, d), "w3": weight(f, d), "w2": weight(d, f)}
+    x = torch.randn((m + 33 + heavy, d), generator=g).to(torch.bfloat16)
+    pd = _blockwise(d) if d <= 2048 else torch.arange(d)
+    pf = _blockwise(f)
+    moved = {"w1": dense["w1"][:, pf][:, :, pd], "w3": dense["w3"][:, pf][:, :, pd],
+             "w2": dense["w2"][:, :, pf]}
+
+    def run(weights, x, n):
+        idx = torch.zeros(n + heavy, 1, dtype=torch.int64)
+        idx[n:] = 1
+        rows = torch.cat([x[:n], x[m + 33:]])
+        with torch.no_grad():
+            return build_module(w, weights, None).run_direct_routed(
+                rows.cuda(), torch.ones(n + heavy, 1, device="cuda"), idx.cuda())[:m]
+
+    few = run(dense, x, m)
+    assert float(few.float().abs().max()) > 0
+    assert torch.equal(few, run(moved, x[:, pd], m + 33))
