@@ -268,8 +268,11 @@ def require_gpu(*tensors: torch.Tensor) -> torch.device:
 
 
 def stream(device: torch.device) -> int:
-    """The current stream's raw handle (without building a torch Stream)."""
-    return torch._C._cuda_getCurrentRawStream(device.index)
+    """The current stream's raw handle (without building a torch Stream). A
+    device without an index is the current one."""
+    index = device.index
+    return torch._C._cuda_getCurrentRawStream(
+        torch.cuda.current_device() if index is None else index)
 
 
 def ptr(t: torch.Tensor | None) -> int | None:

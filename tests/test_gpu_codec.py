@@ -55,6 +55,18 @@ def test_int8_quantize_and_dequantize_bit_exact(shape):
                                   codec.int8_dequantize(q_ref, s_ref))
 
 
+@pytest.mark.parametrize("fmt", ["nf4", "int8", "bf16", "fp32"])
+def test_quantize_takes_a_tensor_in_host_memory(fmt):
+    # The source goes to the current device; the packed weight is the one of a
+    # device tensor.
+    w = _weights((2, 64, 128), seed=13)
+    packed, ref = quant.quantize(w, fmt), quant.quantize(w.cuda(), fmt)
+    assert packed.data.device == ref.data.device
+    assert torch.equal(packed.data, ref.data)
+    if ref.scale is not None:
+        assert torch.equal(packed.scale, ref.scale)
+
+
 def test_fp32_input_is_rounded_to_bf16_first():
     g = torch.Generator().manual_seed(3)
     w32 = torch.randn(2, 32, 256, generator=g) * 0.02
