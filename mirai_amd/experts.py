@@ -105,8 +105,6 @@ class CompressedGroupedExperts(nn.Module):
         self.num_experts = int(num_experts)
         self.mirai_expert_mlp_spec = execution_spec
         self._spec = spec
-        # Tensor names by role (gate, up, down), read on every call.
-        self._roles = tuple(spec.tensor_for_role(r) for r in ("gate", "up", "down"))
         self._group_sizes = group_sizes
         self._quant_format = quant.normalize_quant_format(quant_format)
         self._nf4_blocksize = int(nf4_blocksize)
@@ -329,11 +327,17 @@ class CompressedGroupedExperts(nn.Module):
                 f"compressed_weights grouped experts are missing weights: {missing}.")
 
     def _role_keys(self) -> tuple[str, str, str]:
-        return self._roles
+        # Read on every call: looked up once, also in a module that was pickled
+        # without the names.
+        roles = self.__dict__.get("_roles")
+        if roles is None:
+            roles = self._roles = tuple(self.projection_for_role(r)
+                                        for r in ("gate", "up", "down"))
+        return roles
 
     def _adapters(self) -> list[ActiveExpertLoRA | None]:
         attached = self.expert_lora._modules
-        return [attached.get(k) for k in self._roles]
+        return [attached.get(k) for k in self._role_keys()]
 
     def run_direct_routed(self, tokens: torch.Tensor, top_scores: torch.Tensor,
                           top_indices: torch.Tensor) -> torch.Tensor:

@@ -175,6 +175,22 @@ def test_foreign_spec_objects_are_accepted_by_fields():
         _module(execution_spec=_ForeignSpec(projections=(object(),)))
 
 
+def test_role_names_follow_overrides_and_older_pickles():
+    class Renamed(CompressedGroupedExperts):
+        def projection_for_role(self, role):
+            return {"gate": "w3", "up": "w1", "down": "w2"}[role]
+
+    m = Renamed.from_empty(num_experts=4, quant_format="nf4")
+    assert m._role_keys() == ("w3", "w1", "w2")
+    # A module unpickled from a build that did not keep the names.
+    old = _module()
+    state = {k: v for k, v in old.__dict__.items() if k != "_roles"}
+    new = CompressedGroupedExperts.__new__(CompressedGroupedExperts)
+    new.__setstate__(state)
+    assert new._role_keys() == ("w1", "w3", "w2")
+    assert new._adapters() == [None, None, None]
+
+
 def test_foreign_spec_through_the_base_module_constructor():
     class Base(torch.nn.Module):
         num_experts = 4
