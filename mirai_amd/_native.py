@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import time
 from ctypes import POINTER, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p
 from pathlib import Path
 from typing import Any
@@ -299,19 +300,21 @@ def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
 # (dispatch_preprocess.py:155-157). Reading the counter needs the GPU to have
 # run the plan, so by default ("deferred") each call has it stored into a
 # pinned host slot on its stream (by the layer's plan, or mx_publish_plan_errors)
-# and the count is read once it has landed (counts are not negative, an open slot holds -1): at the
-# start of a later call, or by check_route_errors(), which waits. With "sync"
-# the call itself waits for its plan and raises; "off" skips the store.
+# and the count is read once it has landed (counts are not negative, an open
+# slot holds -1): at the start of a later call, or by check_route_errors(),
+# which waits for the watched plans and nothing else. With "sync" the call
+# itself waits for its plan and raises; "off" skips the store.
 # Calls captured into a HIP graph are not watched.
 ROUTE_CHECK_MODES = ("deferred", "sync", "off")
 _route_check = os.environ.get("MIRAI_ROUTE_CHECK", "deferred").strip().lower()
 if _route_check not in ROUTE_CHECK_MODES:  # pragma: no cover - environment
     _route_check = "deferred"
 _SLOTS = 256
+_ASK_AFTER = 1.0
 _slot_buf: torch.Tensor | None = None  # pinned int32 [_SLOTS]
 _slot_view: Any = None                 # the same memory as a ctypes array
 _slot_next = 0
-_pending: list = []  # (slot index, device, what)
+_pending: list = []  # [slot index, device, stream handle, what (None: read, not reported)]
 
 
 class RouteIndexError(ValueError):
@@ -340,20 +343,41 @@ def _raise_for(count: int, what: str, deferred: bool) -> None:
         f"out of the expert computation.")
 
 
+def _wait_for_slot(slot: int, device: torch.device, handle: int) -> int:
+    """The count of one call, once its plan has stored it. The host memory is
+    watched instead of a stream or device: nothing else the GPU has to do is
+    waited for, and there is no call that a capture on another thread's stream
+    would refuse. Every _ASK_AFTER seconds the call's stream is asked whether it
+    has run out of work without the store."""
+    asked = time.monotonic()
+    while _slot_view[slot] < 0:
+        time.sleep(20e-6)
+        if time.monotonic() - asked > _ASK_AFTER:
+            asked = time.monotonic()
+            s = (torch.cuda.ExternalStream(handle, device=device) if handle
+                 else torch.cuda.default_stream(device))
+            if s.query() and _slot_view[slot] < 0:
+                raise RuntimeError("a plan ended without storing its error count.")
+    return int(_slot_view[slot])
+
+
 def _drain(block: bool) -> None:
     while _pending:
-        slot, device, what = _pending[0]
-        if _slot_view[slot] < 0:
-            if not block:
-                return
-            torch.cuda.synchronize(device)
-        count = int(_slot_view[slot])
-        _pending.pop(0)
-        if count:
-            # No store may still be on its way to a slot given out again.
-            for other in {d for _, d, _ in _pending}:
-                torch.cuda.synchronize(other)
-            _pending.clear()
+        entry = _pending[0]
+        slot, device, handle, what = entry
+        if _slot_view[slot] < 0 and not block:
+            return
+        try:
+            count = _wait_for_slot(slot, device, handle)
+        except RuntimeError:
+            _pending.remove(entry)
+            raise
+        _pending.remove(entry)
+        if count and what is not None:
+            # One report; the counts still on their way are read and dropped,
+            # each before its slot is given out again.
+            for later in _pending:
+                later[3] = None
             _raise_for(count, what, deferred=True)
 
 
@@ -395,13 +419,13 @@ def watch_error_slot(opened: tuple[int, int] | None, device: torch.device, what:
     if opened is None:
         return
     slot = opened[0]
+    handle = stream(device)
     if _route_check == "sync":
-        torch.cuda.current_stream(device).synchronize()
-        count = int(_slot_view[slot])
+        count = _wait_for_slot(slot, device, handle)
         if count:
             _raise_for(count, what, deferred=False)
         return
-    _pending.append((slot, device, what))
+    _pending.append([slot, device, handle, what])
 
 
 def watch_plan_errors(workspace: torch.Tensor, device: torch.device, what: str) -> None:
