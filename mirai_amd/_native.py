@@ -315,6 +315,7 @@ _slot_buf: torch.Tensor | None = None  # pinned int32 [_SLOTS]
 _slot_view: Any = None                 # the same memory as a ctypes array
 _slot_next = 0
 _pending: list = []  # [slot index, device, stream handle, what (None: read, not reported)]
+_dropped: dict = {}  # slot index of a call that failed: (device, stream handle)
 
 
 class RouteIndexError(ValueError):
@@ -343,6 +344,12 @@ def _raise_for(count: int, what: str, deferred: bool) -> None:
         f"out of the expert computation.")
 
 
+def _out_of_work(device: torch.device, handle: int) -> bool:
+    s = (torch.cuda.ExternalStream(handle, device=device) if handle
+         else torch.cuda.default_stream(device))
+    return s.query()
+
+
 def _wait_for_slot(slot: int, device: torch.device, handle: int) -> int:
     """The count of one call, once its plan has stored it. The host memory is
     watched instead of a stream or device: nothing else the GPU has to do is
@@ -354,9 +361,7 @@ def _wait_for_slot(slot: int, device: torch.device, handle: int) -> int:
         time.sleep(20e-6)
         if time.monotonic() - asked > _ASK_AFTER:
             asked = time.monotonic()
-            s = (torch.cuda.ExternalStream(handle, device=device) if handle
-                 else torch.cuda.default_stream(device))
-            if s.query() and _slot_view[slot] < 0:
+            if _out_of_work(device, handle) and _slot_view[slot] < 0:
                 raise RuntimeError("a plan ended without storing its error count.")
     return int(_slot_view[slot])
 
@@ -395,7 +400,7 @@ def check_route_errors() -> None:
 def open_error_slot() -> tuple[int, int] | None:
     """A pinned slot (index, address) for a call's plan error count, or None
     where calls are not watched. watch_error_slot follows once the launch that
-    fills it is queued."""
+    fills it is queued, or drop_error_slot if that fails."""
     global _slot_buf, _slot_view, _slot_next
     # Calls captured into a HIP graph are not watched: a capture may not wait,
     # and a replay would not refresh the slot.
@@ -409,6 +414,10 @@ def open_error_slot() -> tuple[int, int] | None:
     # A slot is reused only after its previous count has been read.
     while any(p[0] == slot for p in _pending):
         _drain(block=True)
+    if slot in _dropped:
+        device, handle = _dropped.pop(slot)
+        while _slot_view[slot] < 0 and not _out_of_work(device, handle):
+            time.sleep(20e-6)
     _slot_view[slot] = -1
     return slot, _slot_buf.data_ptr() + 4 * slot
 
@@ -421,11 +430,23 @@ def watch_error_slot(opened: tuple[int, int] | None, device: torch.device, what:
     slot = opened[0]
     handle = stream(device)
     if _route_check == "sync":
-        count = _wait_for_slot(slot, device, handle)
+        try:
+            count = _wait_for_slot(slot, device, handle)
+        except BaseException:
+            drop_error_slot(opened, device)
+            raise
         if count:
             _raise_for(count, what, deferred=False)
         return
     _pending.append([slot, device, handle, what])
+
+
+def drop_error_slot(opened: tuple[int, int] | None, device: torch.device) -> None:
+    """The call of an opened slot failed. Its plan may have been queued all the
+    same, so the slot is given out again only once the store has landed or the
+    stream is out of work; the count is not reported."""
+    if opened is not None:
+        _dropped[opened[0]] = (device, stream(device))
 
 
 def watch_plan_errors(workspace: torch.Tensor, device: torch.device, what: str) -> None:
@@ -433,5 +454,9 @@ def watch_plan_errors(workspace: torch.Tensor, device: torch.device, what: str) 
     slot by a launch of its own."""
     opened = open_error_slot()
     if opened is not None:
-        call("mx_publish_plan_errors", workspace.data_ptr(), opened[1], stream(device))
+        try:
+            call("mx_publish_plan_errors", workspace.data_ptr(), opened[1], stream(device))
+        except BaseException:
+            drop_error_slot(opened, device)
+            raise
         watch_error_slot(opened, device, what)

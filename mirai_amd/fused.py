@@ -133,12 +133,16 @@ def _forward(module, tokens, top_scores, top_indices, need_grad, addend=None, ad
         addend = addend.contiguous()
     # A call with no tokens builds no plan (and stores no error count).
     slot = nat.open_error_slot() if T > 0 else None
-    nat.call("mx_moe_forward_watched", x.data_ptr(), idx.data_ptr(), scores.data_ptr(),
-             nat.dtype_code(scores.dtype), T, k, E, d, f, kernel_activation(module), w1, w3, w2,
-             lora[0], lora[1], lora[2], out.data_ptr(), nat.dtype_code(out.dtype),
-             nat.ptr(addend), addend_ready.cuda_event if addend_ready is not None else None,
-             *[nat.ptr(t) for t in saves], ws.data_ptr(), slot[1] if slot else None,
-             nat.stream(device))
+    try:
+        nat.call("mx_moe_forward_watched", x.data_ptr(), idx.data_ptr(), scores.data_ptr(),
+                 nat.dtype_code(scores.dtype), T, k, E, d, f, kernel_activation(module), w1, w3,
+                 w2, lora[0], lora[1], lora[2], out.data_ptr(), nat.dtype_code(out.dtype),
+                 nat.ptr(addend), addend_ready.cuda_event if addend_ready is not None else None,
+                 *[nat.ptr(t) for t in saves], ws.data_ptr(), slot[1] if slot else None,
+                 nat.stream(device))
+    except BaseException:
+        nat.drop_error_slot(slot, device)
+        raise
     del keep
     nat.watch_error_slot(slot, device, "a routed expert layer call")
     return out.to(tokens.dtype), ((x, scores, idx, *saves) if need_grad else None)
