@@ -1316,6 +1316,8 @@ template <int FMT>
 constexpr int stream_kstep() {
   return FMT == MX_FMT_BF16 ? 64 : 128;
 }
+// LDS of a stage that takes low-rank rows.
+constexpr int kLoraStage = 32768;
 
 // BLOCKWISE (NF4, one row block): each half-wave multiplies its own 64-block of
 // a step, MFMA step s taking its columns 8 s .. + 7 for weights and tokens
@@ -1414,6 +1416,32 @@ __device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, 
     for (int q = 0; q < kQ; ++q)
       c.q[q] = *reinterpret_cast<const u32x4 *>(codes + static_cast<int64_t>(b) * (2 * kLaneBytes) + kPiece * q);
     c.abs = is_nf4(FMT) ? load_absmax<FMT>(absrow, 2 * b + h) : 0u;
+  };
+
+  // LoRA: the rows' low-rank columns, by DMA after the last K step into the
+  // stage it leaves free, as tiles [MB * 32][32] in the swz64 layout, adapter by
+  // adapter. (Issued inside the step body, it took registers of the K loop.)
+  // Read from global memory in the epilogue they cost a wait per row block,
+  // adapter and 16 columns: layer at rank 64, 72 rows per expert, 128 experts of
+  // hidden 2048 and ffn 768, bf16 454 -> 399 us, INT8 322 -> 290; rank 16 as before.
+  constexpr int n_ad = EPI == EPI_SWIGLU ? 2 : 1;
+  constexpr int kPTile = MB * 32 * 64;
+  static_assert(kLoraStage / kPTile / n_ad >= 2, "64 low-rank columns of each adapter are staged");
+  const int p_tiles = LORA ? min(kLoraStage / kPTile / n_ad, p.lora_rc >> 5) : 0;
+  auto load_p = [&](uint8_t *dst) __attribute__((always_inline)) {
+    constexpr int kDmasPerTile = kPTile / 1024;
+    for (int d = wave; d < n_ad * p_tiles * kDmasPerTile; d += 8) {
+      const int t = d / kDmasPerTile, ad = t >= p_tiles ? 1 : 0, c32 = t - ad * p_tiles;
+      if (pick2(p.lora_r, ad) <= 32 * c32) continue;  // wave-uniform: never multiplied
+      const int pos = (d - t * kDmasPerTile) * 1024 + 16 * lane;
+      const int row = pos >> 6, c = ((pos >> 4) & 3) ^ ((row >> 1) & 3);
+      const int64_t pr = min(row0 + row, row_end - 1);
+      __builtin_amdgcn_global_load_lds(
+          reinterpret_cast<const void *>(p.lora_p + pr * p.ldp + ad * p.lora_rc + 32 * c32 + 8 * c),
+          reinterpret_cast<__attribute__((address_space(3))) void *>(
+              reinterpret_cast<uintptr_t>(dst + d * 1024)),
+          16, 0, 0);
+    }
   };
 
   f32x16 acc[MB];
@@ -1532,33 +1560,67 @@ __device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, 
   }
   if (b < nb) step(b, sA0, sA1, c0, c1);
 
+  // The lane's factor row: its own adapter's (of an absent one the other's, whose
+  // products are not read). Columns past the rank hold zero activations; their
+  // factor read stays inside the row.
+  constexpr int kKeep = 2;  // 16-column steps held over the row blocks
+  int f_r = 0;
+  const uint16_t *frow = nullptr;
+  bf16x8 f_keep[kKeep] = {};
+  const int r_max = !LORA ? 0 : n_ad == 1 ? p.lora_r[0] : max(p.lora_r[0], p.lora_r[1]);
+  uint8_t *sP = (nb & 1) ? sA1 : sA0;  // no wave reads it since the last step's barrier
+  if constexpr (LORA) {
+    const int own = pick2(p.lora_r, which) > 0 ? which : 1 - which;
+    f_r = pick2(p.lora_r, own);
+    frow = pick2(p.lora_b, own) + (static_cast<int64_t>(e) * p.N + n_row) * f_r;
+#pragma unroll
+    for (int s = 0; s < kKeep; ++s)
+      if (16 * s < r_max) {
+        const int col = 16 * s + 8 * h;
+        f_keep[s] = *reinterpret_cast<const bf16x8 *>(frow + (col < f_r ? col : 0));
+      }
+    load_p(sP);
+    wait_lds_dma();
+    __syncthreads();
+  }
+
   // Per row block: the LoRA up-projection, one MFMA chain per adapter. For
   // SwiGLU both chains run over all 32 weight rows of the wave, each lane with
-  // its own column's factor row of the chain's adapter; the gate chain's up
-  // rows (and the reverse) are not read. Then the epilogue: value v of a lane
-  // is output row lane % 32 of the block and weight row 8 (v / 4) + 4 h + v % 4.
-  constexpr int n_ad = EPI == EPI_SWIGLU ? 2 : 1;
+  // its own column's factor row; the gate chain's up rows (and the reverse) are
+  // not read. Then the epilogue: value v of a lane is output row lane % 32 of
+  // the block and weight row 8 (v / 4) + 4 h + v % 4.
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
     const int lrow = 32 * mb + li;
     f32x16 lacc[n_ad];
 #pragma unroll
-    for (int ad = 0; ad < n_ad; ++ad) {
+    for (int ad = 0; ad < n_ad; ++ad)
 #pragma unroll
       for (int j = 0; j < 16; ++j) lacc[ad][j] = 0.0f;
-      if (!LORA) continue;
-      const int r = pick2(p.lora_r, ad);
-      if (r == 0) continue;
-      const int64_t prow_i = min(row0 + lrow, row_end - 1);
-      const uint16_t *frow = pick2(p.lora_b, ad) + (static_cast<int64_t>(e) * p.N + n_row) * r;
-      const uint16_t *arow = p.lora_p + prow_i * p.ldp + ad * p.lora_rc;
-      for (int c = 0; c < r; c += 16) {
+    if constexpr (LORA) {
+      auto staged = [&](int ad, int c) __attribute__((always_inline)) {
+        return *reinterpret_cast<const bf16x8 *>(sP + (ad * p_tiles + (c >> 5)) * kPTile +
+                                                 swz64(lrow, ((c >> 3) & 2) + h));
+      };
+#pragma unroll
+      for (int s = 0; s < kKeep; ++s)
+#pragma unroll
+        for (int ad = 0; ad < n_ad; ++ad)
+          if (16 * s < pick2(p.lora_r, ad))
+            lacc[ad] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f_keep[s], staged(ad, 16 * s),
+                                                               lacc[ad], 0, 0, 0);
+      for (int c = 16 * kKeep; c < r_max; c += 16) {
         const int col = c + 8 * h;
-        // Columns past the rank hold zero activations; their factor read
-        // stays inside the row.
-        const bf16x8 a = *reinterpret_cast<const bf16x8 *>(arow + col);
-        const bf16x8 f = *reinterpret_cast<const bf16x8 *>(frow + (col < r ? col : 0));
-        lacc[ad] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, a, lacc[ad], 0, 0, 0);
+        const bf16x8 f = *reinterpret_cast<const bf16x8 *>(frow + (col < f_r ? col : 0));
+#pragma unroll
+        for (int ad = 0; ad < n_ad; ++ad) {
+          if (c >= pick2(p.lora_r, ad)) continue;
+          const int64_t pr = min(row0 + lrow, row_end - 1);
+          const bf16x8 a = c < 32 * p_tiles ? staged(ad, c)
+                                            : *reinterpret_cast<const bf16x8 *>(
+                                                  p.lora_p + pr * p.ldp + ad * p.lora_rc + col);
+          lacc[ad] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(f, a, lacc[ad], 0, 0, 0);
+        }
       }
     }
     if (lrow >= m) continue;
@@ -1676,7 +1738,8 @@ void grouped_gemm_kernel(Params p) {
 template <int FMT, int EPI, bool LORA>
 __global__ __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(4)))
 void stream_gemm_kernel(Params p) {
-  constexpr int kStage = kPlanTileM * stream_kstep<FMT>() * 2;
+  constexpr int kRows = kPlanTileM * stream_kstep<FMT>() * 2;
+  constexpr int kStage = LORA && kRows < kLoraStage ? kLoraStage : kRows;
   __shared__ __attribute__((aligned(16))) uint8_t sA0[kStage];
   __shared__ __attribute__((aligned(16))) uint8_t sA1[kStage];
   __shared__ float sCode[is_dq(FMT) ? 512 : 1];

@@ -16,7 +16,8 @@ from mirai_amd import workloads as wl
 from oracle import codec
 from oracle import layer as olayer
 
-from helpers import assert_layer_close, build_module, oracle_loras, oracle_weights
+from helpers import (assert_layer_close, build_module, mixed_rank_factors, oracle_loras,
+                     oracle_weights)
 
 pytestmark = pytest.mark.gpu
 
@@ -86,6 +87,26 @@ def test_streaming_tiles(fmt, d, f, rank):
     idx, scores = exact_routes(STREAM_COUNTS, 7)
     dense, x = wl.dense_weights(w), wl.tokens(w)
     lora = wl.lora_factors(w) if rank else None
+    m = build_module(w, dense, lora)
+    with torch.no_grad():
+        out = m.run_direct_routed(x.cuda(), scores.cuda(), idx.cuda())
+    ref = olayer.layer_forward(x, scores, idx, oracle_weights(w, dense), oracle_loras(w, lora),
+                               w.experts)
+    assert_layer_close(out.cpu(), ref)
+
+
+# Low-rank columns staged for the up-projection: 64 of each adapter of gate/up
+# and 128 of down at four row blocks, all 256 at one; further ones
+# are read in the epilogue. Adapters of unequal rank and an absent one too.
+@pytest.mark.parametrize("ranks", [(64, 64, 64), (72, 136, 128), (8, 64, 136), (256, 200, 256),
+                                   (0, 40, 16), (72, 0, 0)])
+@pytest.mark.parametrize("fmt", ["nf4", "bf16"])
+def test_streaming_tiles_of_many_ranks(fmt, ranks):
+    w = workload(fmt, STREAM_COUNTS, d=256, f=384)
+    idx, scores = exact_routes(STREAM_COUNTS, 9)
+    dense, x = wl.dense_weights(w), wl.tokens(w)
+    lora = mixed_rank_factors(w, dict(zip(("w1", "w3", "w2"), (max(r, 1) for r in ranks))))
+    lora = {key: t for (key, t), r in zip(lora.items(), ranks) if r}
     m = build_module(w, dense, lora)
     with torch.no_grad():
         out = m.run_direct_routed(x.cuda(), scores.cuda(), idx.cuda())
