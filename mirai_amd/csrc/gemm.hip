@@ -1336,8 +1336,28 @@ __device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, 
   const int64_t row0 = tile.y;
   const int64_t row_end = p.seg_end[e];
   const int m = static_cast<int>(min(row_end - row0, static_cast<int64_t>(MB * 32)));
-  const int wave = uniform_wave_index(), lane = threadIdx.x & 63;
-  const int li = lane & 31, h = lane >> 5;
+  const int wave = uniform_wave_index();
+
+  // The lane's weight row, of the tile's 256.
+  int lane, li, h, which = 0;
+  int64_t n_row;
+  auto lane_row = [&](int l) __attribute__((always_inline)) {
+    lane = l;
+    li = l & 31;
+    h = l >> 5;
+    int64_t n;
+    if (EPI == EPI_SWIGLU) {
+      // Rows 0..15 of the wave's block: gate rows of ffn columns f0 .. f0 + 15;
+      // rows 16..31: the up rows of the same columns, so value v and v + 8 of a
+      // lane's accumulator are one (gate, up) pair.
+      which = li >> 4;
+      n = static_cast<int64_t>(nt) * 128 + 16 * wave + (li & 15);
+    } else {
+      n = static_cast<int64_t>(nt) * 256 + 32 * wave + li;
+    }
+    n_row = min(n, p.N - 1);  // rows past N feed dropped columns
+  };
+  lane_row(threadIdx.x & 63);
 
   // ------------------------------------------- token rows -> LDS (by DMA)
   // 16-byte chunks of a staged row XOR-ed with a row key, so the 32 rows of a
@@ -1366,18 +1386,6 @@ __device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, 
   };
 
   // ----------------------------------------------------- the wave's weights
-  int which = 0;
-  int64_t n;
-  if (EPI == EPI_SWIGLU) {
-    // Rows 0..15 of the wave's block: gate rows of ffn columns f0 .. f0 + 15;
-    // rows 16..31: the up rows of the same columns, so value v and v + 8 of a
-    // lane's accumulator are one (gate, up) pair.
-    which = li >> 4;
-    n = static_cast<int64_t>(nt) * 128 + 16 * wave + (li & 15);
-  } else {
-    n = static_cast<int64_t>(nt) * 256 + 32 * wave + li;
-  }
-  const int64_t n_row = min(n, p.N - 1);  // rows past N feed dropped columns
   const int64_t wrow = static_cast<int64_t>(e) * pick(p.wn, which) + n_row;
   // Bytes of one lane's share of a step, its 16-byte registers and the row's
   // bytes per step.
@@ -1416,32 +1424,6 @@ __device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, 
     for (int q = 0; q < kQ; ++q)
       c.q[q] = *reinterpret_cast<const u32x4 *>(codes + static_cast<int64_t>(b) * (2 * kLaneBytes) + kPiece * q);
     c.abs = is_nf4(FMT) ? load_absmax<FMT>(absrow, 2 * b + h) : 0u;
-  };
-
-  // LoRA: the rows' low-rank columns, by DMA after the last K step into the
-  // stage it leaves free, as tiles [MB * 32][32] in the swz64 layout, adapter by
-  // adapter. (Issued inside the step body, it took registers of the K loop.)
-  // Read from global memory in the epilogue they cost a wait per row block,
-  // adapter and 16 columns: layer at rank 64, 72 rows per expert, 128 experts of
-  // hidden 2048 and ffn 768, bf16 454 -> 399 us, INT8 322 -> 290; rank 16 as before.
-  constexpr int n_ad = EPI == EPI_SWIGLU ? 2 : 1;
-  constexpr int kPTile = MB * 32 * 64;
-  static_assert(kLoraStage / kPTile / n_ad >= 2, "64 low-rank columns of each adapter are staged");
-  const int p_tiles = LORA ? min(kLoraStage / kPTile / n_ad, p.lora_rc >> 5) : 0;
-  auto load_p = [&](uint8_t *dst) __attribute__((always_inline)) {
-    constexpr int kDmasPerTile = kPTile / 1024;
-    for (int d = wave; d < n_ad * p_tiles * kDmasPerTile; d += 8) {
-      const int t = d / kDmasPerTile, ad = t >= p_tiles ? 1 : 0, c32 = t - ad * p_tiles;
-      if (pick2(p.lora_r, ad) <= 32 * c32) continue;  // wave-uniform: never multiplied
-      const int pos = (d - t * kDmasPerTile) * 1024 + 16 * lane;
-      const int row = pos >> 6, c = ((pos >> 4) & 3) ^ ((row >> 1) & 3);
-      const int64_t pr = min(row0 + row, row_end - 1);
-      __builtin_amdgcn_global_load_lds(
-          reinterpret_cast<const void *>(p.lora_p + pr * p.ldp + ad * p.lora_rc + 32 * c32 + 8 * c),
-          reinterpret_cast<__attribute__((address_space(3))) void *>(
-              reinterpret_cast<uintptr_t>(dst + d * 1024)),
-          16, 0, 0);
-    }
   };
 
   f32x16 acc[MB];
@@ -1559,6 +1541,38 @@ __device__ __forceinline__ void stream_tile(const Params &p, int2 tile, int nt, 
     step(b + 1, sA1, sA0, c1, c0);
   }
   if (b < nb) step(b, sA0, sA1, c0, c1);
+
+  // The lane's indices again, opaque, so that what the epilogue derives from them
+  // holds no registers over the K loop.
+  int tid = threadIdx.x;
+  asm volatile("" : "+v"(tid));
+  lane_row(tid & 63);
+
+  // LoRA: the rows' low-rank columns, by DMA after the last K step into the
+  // stage it leaves free, as tiles [MB * 32][32] in the swz64 layout, adapter by
+  // adapter. (Issued inside the step body, it took registers of the K loop.)
+  // Read from global memory in the epilogue they cost a wait per row block,
+  // adapter and 16 columns: layer at rank 64, 72 rows per expert, 128 experts of
+  // hidden 2048 and ffn 768, bf16 454 -> 399 us, INT8 322 -> 290; rank 16 as before.
+  constexpr int n_ad = EPI == EPI_SWIGLU ? 2 : 1;
+  constexpr int kPTile = MB * 32 * 64;
+  static_assert(kLoraStage / kPTile / n_ad >= 2, "64 low-rank columns of each adapter are staged");
+  const int p_tiles = LORA ? min(kLoraStage / kPTile / n_ad, p.lora_rc >> 5) : 0;
+  auto load_p = [&](uint8_t *dst) __attribute__((always_inline)) {
+    constexpr int kDmasPerTile = kPTile / 1024;
+    for (int d = wave; d < n_ad * p_tiles * kDmasPerTile; d += 8) {
+      const int t = d / kDmasPerTile, ad = t >= p_tiles ? 1 : 0, c32 = t - ad * p_tiles;
+      if (pick2(p.lora_r, ad) <= 32 * c32) continue;  // wave-uniform: never multiplied
+      const int pos = (d - t * kDmasPerTile) * 1024 + 16 * lane;
+      const int row = pos >> 6, c = ((pos >> 4) & 3) ^ ((row >> 1) & 3);
+      const int64_t pr = min(row0 + row, row_end - 1);
+      __builtin_amdgcn_global_load_lds(
+          reinterpret_cast<const void *>(p.lora_p + pr * p.ldp + ad * p.lora_rc + 32 * c32 + 8 * c),
+          reinterpret_cast<__attribute__((address_space(3))) void *>(
+              reinterpret_cast<uintptr_t>(dst + d * 1024)),
+          16, 0, 0);
+    }
+  };
 
   // The lane's factor row: its own adapter's (of an absent one the other's, whose
   // products are not read). Columns past the rank hold zero activations; their
