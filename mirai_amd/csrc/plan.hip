@@ -9,7 +9,7 @@
 // Pass 1 writes per-block expert counts (and per-block counts of invalid ids),
 // pass 2 scans them into per-(block, expert) bases and writes the plan's error
 // count, pass 3 rebuilds the masks and scatters. Passes 2 and 3 are one kernel
-// up to 1024 experts and 65536 block counts, all three are one where a single
+// up to 1024 experts, 65536 block counts and 2048 blocks, all three are one where a single
 // block takes the slots, and pass 2 is a launch of one workgroup otherwise.
 // Every counter is written, not accumulated, so a plan needs no clearing launch.
 #include "common.h"
@@ -339,6 +339,11 @@ __device__ __forceinline__ void wg_exclusive_scan(const int32_t (&v)[N], int32_t
 // most) 30.4 -> 20.7; 98304 slots of 128 experts 27.8 -> 18.8. (With 64-bit scans unrolled over the
 // waves the kernel spilled, and took 12.7 us for the 64 slots.)
 constexpr int kFusedCounts = 65536;
+// And at most so many blocks: each reads the counts of all, blocks^2 * experts
+// counts together. Plan call with 4 and 8 experts, three kernels against this: 2048
+// blocks (8388608 slots) 1226 / 1170 and 739 / 706 us, 4096 blocks 2376 / 2476 and
+// 1450 / 1492.
+constexpr int kFusedBlocks = 2048;
 // Mask bits (E * EB) of a block: masks and prefixes take 32 KB of LDS.
 constexpr int kFusedBits = 131072;
 
@@ -582,7 +587,7 @@ int build_plan(const int64_t *top_idx, const void *top_scores, int score_dtype,
   }
   // The fused kernel takes one expert per thread.
   if (eb1 > 0 || (L.blocks > 1 && num_experts <= 1024 &&
-                  num_experts * L.slots_per_block <= kFusedBits &&
+                  num_experts * L.slots_per_block <= kFusedBits && L.blocks <= kFusedBlocks &&
                   static_cast<int64_t>(L.blocks) * num_experts <= kFusedCounts)) {
     PlanFused a = {};
     a.top_idx = top_idx;

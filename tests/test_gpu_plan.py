@@ -65,6 +65,7 @@ def test_plan_random_with_duplicates_and_invalid_ids(T, k, E):
     (129, 1024),              # one block, or just too many slots or mask bits for one
     (65536, 128), (65537, 128),  # 256 blocks of 128 experts, and one more block
     (65536, 256), (65537, 256),  # 65536 block counts, and 256 more
+    (8388608, 4), (8388609, 4),  # 2048 blocks, and one more
     (20000, 1000), (3000, 65), (600, 2)])
 def test_plan_block_edges(R, E):
     """Sizes on both sides of the rules that pick one block, fused or separate
@@ -81,6 +82,29 @@ def test_plan_block_edges(R, E):
     dropped = build_dispatch_plan(torch.from_numpy(ids).cuda(), torch.from_numpy(scores).cuda(), E)
     for field in ("counts", "starts", "offsets", "inverse_order"):
         assert torch.equal(getattr(plan, field), getattr(dropped, field))
+
+
+@pytest.mark.parametrize("R,E", [(31, 64), (2048, 64), (2049, 64), (4097, 32), (65536, 256),
+                                 (65537, 256), (20000, 1000), (3000, 1100)])
+def test_plan_error_counts(R, E, monkeypatch):
+    """Ids outside the range are counted whichever kernels build the plan, and
+    dropped slots are not."""
+    from mirai_amd import _native as nat
+
+    made = []
+    workspace = nat.workspace
+    monkeypatch.setattr(nat, "workspace", lambda *a: made.append(workspace(*a)) or made[-1])
+    idx = torch.arange(R).view(R, 1) % E
+    scores = torch.ones(R, 1)
+    for wrong, count in ((E, len(range(3, R, 50))), (-1, len(range(3, R, 50))),
+                         (nat.ROUTE_DROPPED, 0)):
+        ids = idx.clone()
+        ids[3::50, 0] = wrong
+        ids[R // 2, 0] = nat.ROUTE_DROPPED
+        build_dispatch_plan(ids.cuda(), scores.cuda(), E)
+        if wrong != nat.ROUTE_DROPPED and R // 2 % 50 == 3:
+            count -= 1
+        assert int(made[-1][:4].view(torch.int32)) == count
 
 
 def test_plan_bf16_scores_and_zero_tokens():
