@@ -451,6 +451,18 @@ int mx_set_stage_events(void **events, int count);
 size_t mx_moe_workspace_size(int64_t num_tokens, int top_k, int num_experts,
                              int64_t hidden, int64_t ffn, int lora_rank);
 
+/*
+ * How a grouped GEMM over weights of `format` is tiled: K weight columns per
+ * output (hidden for gate/up, ffn for down; three times those for MX_FMT_F32X3),
+ * `rows` routed rows over `experts` experts; backward != 0: the GEMMs through
+ * the weights' columns. For tests and profiles: results do not depend on it
+ * beyond the order of fp32 sums.
+ */
+#define MX_LAUNCH_128 0    /* 128-row tiles that stage decoded weights */
+#define MX_LAUNCH_STREAM 1 /* weight-streaming tiles of at most 128 rows */
+#define MX_LAUNCH_DUAL 2   /* 256-row tiles and remainders of at most 128 rows */
+int mx_gemm_launch(int format, int backward, int64_t K, int64_t rows, int experts);
+
 /* Bytes of scratch for mx_moe_forward with MX_FMT_F32X3 weights (fp32 tokens). */
 size_t mx_moe_f32x3_workspace_size(int64_t num_tokens, int top_k, int num_experts,
                                    int64_t hidden, int64_t ffn);

@@ -34,6 +34,10 @@ FMT_NF4_F32_KN = 5  # the same, stored [E, in, out] with the blocks along out (M
 FMT_NF4_DQ = 6     # NF4 codes with a bitsandbytes two-level absmax decoded in the GEMMs
 FMT_NF4_DQ_KN = 7  # the same, stored [E, in, out]
 
+LAUNCH_128 = 0     # mx_gemm_launch: how a grouped GEMM is tiled
+LAUNCH_STREAM = 1
+LAUNCH_DUAL = 2
+
 SPLIT_ACT = 0      # mx_split_f32 plane orders
 SPLIT_WEIGHT = 1
 
@@ -157,6 +161,7 @@ SIGNATURES: dict[str, tuple[Any, list[Any]]] = {
     "mx_int8_dequantize": (c_int, [_P, _P, c_int64, c_int64, _P, c_int, _P]),
     "mx_set_stage_events": (c_int, [POINTER(c_void_p), c_int]),
     "mx_moe_workspace_size": (c_size_t, [c_int64, c_int, c_int, c_int64, c_int64, c_int]),
+    "mx_gemm_launch": (c_int, [c_int, c_int, c_int64, c_int64, c_int]),
     "mx_moe_f32x3_workspace_size": (c_size_t, [c_int64, c_int, c_int, c_int64, c_int64]),
     "mx_split_f32": (c_int, [_P, c_int64, c_int64, c_int, _P, _P]),
     "mx_moe_forward": (

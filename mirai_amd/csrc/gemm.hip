@@ -1871,18 +1871,28 @@ int launch_dual(const Params &p, int64_t max_tall, int64_t max_short, hipStream_
 // Whether a launch takes the dual kernel (256-row tiles, remainders of at most
 // 128 rows) or 128-row tiles alone: by the rows per expert on average.
 // * The forward over NF4, INT8 and bf16 weights (`stream`): the 128-row tiles
-//   are weight-streaming tiles at two workgroups per CU. Layers of 64 or 128
-//   experts, streaming against dual: INT8 at 24 rows per expert 328 / 369 us, 48
-//   382 / 412, 56 458 / 439; NF4 at 32 182 / 248, at 64 247 / 263 with even
-//   routes but 265 / 242 skewed (heavy experts want tall tiles): 48. bf16
-//   weights are four times the bytes to wait for, and the second workgroup
-//   pays longer: at 80 344 / 374, at 112 409 / 409. With few K steps a tile is
+//   are weight-streaming tiles at two workgroups per CU. Layers (us), streaming /
+//   dual, even routes, then skewed ones (heavy experts want tall tiles):
+//     rows per expert        32                48                64
+//     NF4  2048 x 1408   169/178 163/145   196/202 170/149   228/229 201/178
+//     INT8 2048 x 1408   180/195 170/145   215/205 173/154   238/223 203/182
+//     NF4  3072 x 2048   302/318 260/247   346/365 297/277   405/420 354/330
+//     INT8 3072 x 2048   340/354 284/256   384/381 315/274   470/410 401/326
+//   so 48. bf16 weights are four times the bytes to wait for, and the second
+//   workgroup pays longer: 2048 x 1408 at 80 325/348 281/274, 104 337/362 329/325,
+//   116 420/372 339/328; 128 experts of ffn 768 at 116 456/481 359/351: 112. (With
+//   even routes the tiles that stage weights are better than both between about
+//   96 and 120 rows of bf16, by at most 6 %; with skewed ones worse than both by up
+//   to 20 %, and the rule does not see the routes.) With few K steps a tile is
 //   mostly its start and end, which the second workgroup covers: K = 256 and
-//   512, 256 experts, at 150 142 / 161, 256 196 / 210, INT8 at 300 242 / 236.
+//   512, 256 experts, at 150 142/161, 256 196/210; at K = 512 and 768 NF4 at 110
+//   62/69 63/72, 200 80/85; at K = 640 the two are equal from 48 with even routes,
+//   and skewed ones stay better streamed up to about 96 (55/64 at 56).
 // * Otherwise both launches cover up to 128 rows with the same tile, and a
 //   tall tile decodes the weights of 129 or more rows once instead of twice:
-//   from 32 rows per expert on the dual launch was never slower, below that few
-//   experts exceed 128 rows and its empty workgroups cost more.
+//   training steps from 32 rows per expert on are 0.98 to 1.2 times as fast with
+//   the dual launch, the more the more rows; below that few experts exceed 128
+//   rows and its empty workgroups cost more.
 // * The fp32 layer keeps 256: its down projection's K parts belong to the
 //   128-row launch.
 inline bool use_tall_tiles(int fmt, bool stream, int64_t K, int64_t rows, int experts) {
@@ -1892,6 +1902,15 @@ inline bool use_tall_tiles(int fmt, bool stream, int64_t K, int64_t rows, int ex
                         : fmt == MX_FMT_BF16 ? 112
                                              : 48;
   return rows >= least * static_cast<int64_t>(experts);
+}
+
+// The launch of a grouped GEMM with K weight columns per output over `rows` rows
+// (backward: the GEMMs through the weights' columns, EPI_STORE2).
+inline int gemm_launch(int fmt, bool backward, int64_t K, int64_t rows, int experts) {
+  const bool stream = !backward && stream_format(fmt) && K % 128 == 0;
+  // The backward has no 256-row tile over two-level absmax.
+  const bool tall = !(backward && is_dq(fmt)) && use_tall_tiles(fmt, stream, K, rows, experts);
+  return tall ? MX_LAUNCH_DUAL : stream ? MX_LAUNCH_STREAM : MX_LAUNCH_128;
 }
 
 // fp32 layer, down projection on 128-row tiles: K parts per tile, so that a
@@ -1996,15 +2015,13 @@ int launch_fmt(int fmt, Params p, const PlanLayout &PL, const PlanView &v, hipSt
                                          Tile<256, 256, 2, 4, 64>>::type;
   using Short = Tile<128, 256, 2, 4, 64>;
   p.n_tiles_n = static_cast<int>(EPI == EPI_SWIGLU ? ceil_div(p.N, 128) : ceil_div(p.N, 256));
-  const bool stream = EPI != EPI_STORE2 && stream_format(fmt) && p.K % 128 == 0;
-  bool tall = use_tall_tiles(fmt, stream, p.K, PL.rows, PL.experts);
-  if (EPI == EPI_STORE2 && (fmt == MX_FMT_NF4_DQ || fmt == MX_FMT_NF4_DQ_KN)) tall = false;
-  if (!tall) {
+  const int kind = gemm_launch(fmt, EPI == EPI_STORE2, p.K, PL.rows, PL.experts);
+  if (kind != MX_LAUNCH_DUAL) {
     p.tiles = v.tiles;
     p.num_tiles = v.num_tiles;
     const int64_t max_tiles = std::min(PL.max_tiles, PL.rows);
     if constexpr (EPI == EPI_SWIGLU || EPI == EPI_STORE)
-      if (stream) return launch_stream_fmt<EPI, LORA>(fmt, p, max_tiles, s);
+      if (kind == MX_LAUNCH_STREAM) return launch_stream_fmt<EPI, LORA>(fmt, p, max_tiles, s);
     return launch_tile<EPI, LORA, Short>(fmt, p, max_tiles, s);
   }
   // 256-row tiles over each expert's rows except a final remainder of at most
@@ -2879,6 +2896,10 @@ extern "C" size_t mx_moe_workspace_size(int64_t num_tokens, int top_k, int num_e
     return 0;
   return layer_layout(num_tokens * top_k, num_experts, hidden, ffn, false, 0,
                       lora_width(lora_rank)).bytes;
+}
+
+extern "C" int mx_gemm_launch(int format, int backward, int64_t K, int64_t rows, int experts) {
+  return gemm_launch(format, backward != 0, K, rows, experts);
 }
 
 extern "C" size_t mx_moe_f32x3_workspace_size(int64_t num_tokens, int top_k, int num_experts,

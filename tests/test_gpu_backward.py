@@ -8,10 +8,11 @@ the bf16 reference composition does, but the reference's autograd also sums
 the k routes of a token and the base/LoRA parts of each gradient in bf16, in
 an order torch does not fix. Bounds (stated per gradient, relative to the
 oracle): mean-relative error <= 5e-3 and max-abs error <= 3e-2 * max|oracle|.
-Production tile shapes: experts averaging >= 256 rows run 256-row tiles plus
-one 128-row remainder tile per expert whose last rows number 1..128 (an
-expert whose last rows number 129..255 gets a partial 256-row tile). The
-tall-tile cases below meet that threshold and assert which tiles they cover;
+Production tile shapes: where mx_gemm_launch says so (the backward's GEMMs
+from 32 rows per expert on, the forward's from 48 to 256) experts run 256-row
+tiles plus one 128-row remainder tile per expert whose last rows number 1..128
+(an expert whose last rows number 129..255 gets a partial 256-row tile). The
+tall-tile cases below average at least 256 rows and assert which tiles they cover;
 full C5 runs on every token (so on the production tiles) and is compared with
 the oracle on a token subset for d tokens / d scores, and per expert for the
 LoRA gradients (an expert's LoRA gradients sum only its own rows, so the
@@ -23,6 +24,7 @@ scales every gradient by exactly 2) and run-to-run determinism.
 import pytest
 import torch
 
+from mirai_amd import _native as nat
 from mirai_amd import workloads as wl
 from oracle import layer as olayer
 from oracle import routing as oroute
@@ -150,7 +152,8 @@ def _tile_kinds(idx, E):
     """(tall tiles used, experts with a 128-row remainder tile, experts whose
     last rows need a partial 256-row tile) -- the plan's tile rule."""
     counts = torch.bincount(idx.reshape(-1), minlength=E)
-    tall = int(counts.sum()) >= 256 * E
+    tall = nat.load_library().mx_gemm_launch(nat.FMT_NF4, 1, 256, int(counts.sum()),
+                                             E) == nat.LAUNCH_DUAL
     rem = counts % 256
     return tall, int(((rem > 0) & (rem <= 128)).sum()), int((rem > 128).sum())
 

@@ -1,14 +1,15 @@
-"""GPU parity of the light tiles against the reference-order oracle.
+"""GPU parity of experts with few rows against the reference-order oracle.
 
-An expert with at most 32 rows in a launch runs a tile body of its own: its
-token rows are staged in LDS once and each wave decodes its NF4 weight rows
-straight into MFMA operands (no per-step B stage). The cases below route
-exact row counts to chosen experts (0, 1, 5, 16, 31, 32 and 33 rows: both
-sides of the threshold), next to heavy experts that keep the 256-row tiles
-running in the same launch, or with few rows overall (128-row tile launch).
-Both GEMMs take the light body when their K is a multiple of 128 (d = 256,
-f = 384 here). Bounds: the layer bound of test_gpu_layer.py forward, the
-per-gradient bounds of test_gpu_backward.py for training.
+In the forward such experts run weight-streaming tiles: each wave decodes its
+own weight rows straight into MFMA operands and the token rows go through LDS
+step by step, for 1, 2 or 4 blocks of 32 rows. NF4 tiles of one block sum K in
+an order of their own. The cases below route exact row counts to chosen experts
+(0, 1, 5, 16, 31, 32 and 33 rows: both sides of the first block), next to heavy
+experts that keep the 256-row tiles running in the same launch, or with few
+rows overall (the streaming launch). Both GEMMs stream when their K is a
+multiple of 128 (d = 256, f = 384 here). Bounds: the layer bound of
+test_gpu_layer.py forward, the per-gradient bounds of test_gpu_backward.py for
+training.
 """
 
 import numpy as np
