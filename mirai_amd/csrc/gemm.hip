@@ -1287,17 +1287,23 @@ __device__ __forceinline__ void gemm_tile(Params p, int2 tile, int nt, uint8_t *
 
 // ------------------------------------------------- weight-streaming tiles
 // Forward tiles of at most 128 rows (few rows per expert, remainders): the
-// weights are the work there, each is decoded once, and what bounds the tile
-// is the decode's VALU and the wait for the next weights, not MFMA. So each
+// weights are the work there, each is decoded once, and the tile takes its time
+// from the decode's VALU and the waits between it, not from MFMA. So each
 // wave decodes its own 32 weight rows straight into MFMA operands and holds
 // every row block's accumulators (MB = 1, 2 or 4 blocks of 32 rows): no B
-// stage, and one barrier per 128 columns of K, for the token rows that all
-// waves share through LDS. With 64 KB of LDS and 128 registers two workgroups
-// run on a CU, four waves per SIMD, and cover each other's waits; the tile that
-// stages decoded weights in LDS runs one, and a barrier per 64 columns.
+// stage, and one barrier per 128 columns of K (bf16 weights: 64), for the token
+// rows that all waves share through LDS. With 64 KB of LDS (bf16 without LoRA:
+// 32) and 128 registers two workgroups run on a CU, four waves per SIMD, and
+// cover each other's waits; the tile that stages decoded weights in LDS runs one,
+// and a barrier per 64 columns. In 128 registers the four-block bodies of INT8
+// and two-level NF4 reload 3 or 4 spilled ones per two K steps; the others spill
+// nothing inside their K loops.
 // Measured (kernel trace, hidden 2048, ffn 1408, 64 NF4 experts): gate/up at 256
 // tokens 82 -> 69 us (2.8 TB/s of packed weights), at 512 tokens 130 -> 80; INT8,
-// hidden 3072, ffn 2048, 300 tokens: the layer 474 -> 324 us (4.5 TB/s). Weights
+// hidden 3072, ffn 2048, 300 tokens: the layer 474 -> 324 us (1.21 GB of weights,
+// 3.7 TB/s over the whole layer). Counters at 256 tokens, gate/up and down: VALU
+// issue 76 and 69 % of the busy CUs' cycles, MFMA 18 and 16 %, a wave waits 45 and
+// 48 % of its time; at 16 tokens 77 and 65 %, 18 and 15 %, 43 and 47 %. Weights
 // loaded two or three steps ahead instead of one: slower (300 tokens INT8 324 ->
 // 348 us, 256 tokens NF4 163 -> 171).
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
