@@ -9,6 +9,7 @@ from __future__ import annotations
 
 import ctypes
 import os
+import threading
 import time
 from ctypes import POINTER, c_float, c_int, c_int32, c_int64, c_size_t, c_void_p
 from pathlib import Path
@@ -319,6 +320,8 @@ _ASK_AFTER = 1.0
 _slot_buf: torch.Tensor | None = None  # pinned int32 [_SLOTS]
 _slot_view: Any = None                 # the same memory as a ctypes array
 _slot_next = 0
+_slot_lock = threading.Lock()   # handing out slots
+_drain_lock = threading.Lock()  # reading pending ones
 _pending: list = []  # [slot index, device, stream handle, what (None: read, not reported)]
 _dropped: dict = {}  # slot index of a call that failed: (device, stream handle)
 
@@ -372,23 +375,28 @@ def _wait_for_slot(slot: int, device: torch.device, handle: int) -> int:
 
 
 def _drain(block: bool) -> None:
-    while _pending:
-        entry = _pending[0]
-        slot, device, handle, what = entry
-        if _slot_view[slot] < 0 and not block:
-            return
-        try:
-            count = _wait_for_slot(slot, device, handle)
-        except RuntimeError:
-            _pending.remove(entry)
-            raise
-        _pending.remove(entry)
-        if count and what is not None:
-            # One report; the counts still on their way are read and dropped,
-            # each before its slot is given out again.
-            for later in _pending:
-                later[3] = None
-            _raise_for(count, what, deferred=True)
+    # One thread reads at a time; a call that does not wait leaves it to that one.
+    if not _drain_lock.acquire(blocking=block):
+        return
+    try:
+        while _pending:
+            slot, device, handle, what = _pending[0]
+            if _slot_view[slot] < 0 and not block:
+                return
+            try:
+                count = _wait_for_slot(slot, device, handle)
+            except RuntimeError:
+                _pending.pop(0)
+                raise
+            _pending.pop(0)
+            if count and what is not None:
+                # One report; the counts still on their way are read and dropped,
+                # each before its slot is given out again.
+                for later in _pending:
+                    later[3] = None
+                _raise_for(count, what, deferred=True)
+    finally:
+        _drain_lock.release()
 
 
 def poll_route_errors() -> None:
@@ -411,11 +419,13 @@ def open_error_slot() -> tuple[int, int] | None:
     # and a replay would not refresh the slot.
     if _route_check == "off" or torch.cuda.is_current_stream_capturing():
         return None
-    if _slot_buf is None:
-        _slot_buf = torch.full((_SLOTS,), -1, dtype=torch.int32, pin_memory=True)
-        _slot_view = (c_int32 * _SLOTS).from_address(_slot_buf.data_ptr())
-    slot = _slot_next
-    _slot_next = (_slot_next + 1) % _SLOTS
+    with _slot_lock:
+        if _slot_buf is None:
+            buf = torch.full((_SLOTS,), -1, dtype=torch.int32, pin_memory=True)
+            _slot_view = (c_int32 * _SLOTS).from_address(buf.data_ptr())
+            _slot_buf = buf
+        slot = _slot_next
+        _slot_next = (_slot_next + 1) % _SLOTS
     # A slot is reused only after its previous count has been read.
     while any(p[0] == slot for p in _pending):
         _drain(block=True)

@@ -341,3 +341,36 @@ def test_route_check_modes():
         nat.set_route_check("loud")
     assert issubclass(nat.RouteIndexError, ValueError)
     nat.check_route_errors()  # nothing pending: returns
+
+
+def test_threads_wait_for_route_counts_together(monkeypatch):
+    # Four threads wait for the same three counts, which land one by one: each
+    # returns, one of them with the report of the second.
+    import ctypes
+    import threading
+    import time
+
+    slots = (ctypes.c_int32 * 3)(-1, -1, -1)
+    monkeypatch.setattr(nat, "_slot_view", slots)
+    monkeypatch.setattr(nat, "_pending", [[i, torch.device("cpu"), 0, f"call {i}"] for i in range(3)])
+    outcome = []
+
+    def check():
+        try:
+            nat.check_route_errors()
+            outcome.append(None)
+        except Exception as err:  # noqa: BLE001 - recorded for the assertion
+            outcome.append(err)
+
+    threads = [threading.Thread(target=check) for _ in range(4)]
+    for t in threads:
+        t.start()
+    for i, count in enumerate((0, 5, 0)):
+        time.sleep(0.02)
+        slots[i] = count
+    for t in threads:
+        t.join(timeout=10)
+    assert len(outcome) == 4 and not nat._pending
+    errors = [e for e in outcome if e is not None]
+    assert len(errors) == 1 and isinstance(errors[0], nat.RouteIndexError)
+    assert str(errors[0]).startswith("5 route slot")
