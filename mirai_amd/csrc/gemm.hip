@@ -1832,6 +1832,9 @@ void grouped_gemm_dual_kernel(Params p) {
     // The forward's remainder tiles stream their weights too (top-8 of 128
     // experts, skewed: 8192 tokens 896 -> 878 us, INT8 3000 tokens 730 -> 682).
     if constexpr (stream_capable<FMT, EPI>()) {
+      static_assert(Tall::STAGE_A >= kPlanTileM * stream_kstep<FMT>() * 2 &&
+                        (!LORA || Tall::STAGE_A >= kLoraStage),
+                    "a streaming stage must fit the tall tile's");
       if (p.K % 128 == 0) {
         stream_rows<FMT, EPI, LORA>(p, tile, logical - mt * p.n_tiles_n, sA0, sA1, sCode);
         return;
